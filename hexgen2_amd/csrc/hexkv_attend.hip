@@ -60,6 +60,7 @@
 //     form reads stale data: the XCDs' L2s are not coherent.)
 //   * otherwise `combine_kernel`, launched next on the same stream.
 #include "hexkv_common.h"
+#include "hexkv_prefill.h"
 
 #include <algorithm>
 #include <atomic>
@@ -243,20 +244,6 @@ __device__ __forceinline__ bool begin_work(const AttendArgs &a, Work &w) {
 // Largest partition count a single-launch merge takes (the host sends calls
 // with more to combine_kernel): one wave holds a head's (max, sum) pairs.
 constexpr int kMergeMaxParts = 64;  // also keeps each XCD's 8-bit arrival count from overflowing
-
-// Four consecutive outputs at p, one vector store when p is aligned for it
-// (output rows may have any element stride).
-template <typename T>
-__device__ __forceinline__ void store4(T *p, f32x4 v) {
-  if ((reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0) {
-    typedef T t4 __attribute__((ext_vector_type(4)));
-    *reinterpret_cast<t4 *>(p) = t4{Elem<T>::from_float(v[0]), Elem<T>::from_float(v[1]),
-                                    Elem<T>::from_float(v[2]), Elem<T>::from_float(v[3])};
-  } else {
-#pragma unroll
-    for (int k = 0; k < 4; ++k) p[k] = Elem<T>::from_float(v[k]);
-  }
-}
 
 // The XCD-local merge of a split segment (row, head group qh0 / G), after
 // this workgroup stored its partial: count the arrival; the last of the
@@ -1521,6 +1508,32 @@ static int choose_partition(const hexkv_attend_params *p) {
   return part;
 }
 
+// Whether a call runs the query-tile kernel (hexkv_prefill.hip): several
+// query rows per sequence, AUTO, 16-bit data of head_dim 64 or 128.  An
+// explicit VALU or MFMA request keeps the per-row kernel it names.
+static bool use_tiles(const hexkv_attend_params *p) {
+  return p->q_len > 1 && p->kernel == HEXKV_KERNEL_AUTO && tiles_support(p->dtype, p->head_dim);
+}
+
+// Partition size of a tile call: all keys in one partition once the tiles
+// fill the CUs, else enough partitions for about 512 workgroups.  Never
+// below the per-row kernels' partition, so no call needs more workspace
+// than it did with one.
+static int tile_partition(const hexkv_attend_params *p) {
+  const int per_row = choose_partition(p);
+  if (p->partition > 0) return per_row;
+  const int64_t rows = static_cast<int64_t>(p->q_len) * (p->q_heads / p->kv_heads);
+  const int64_t per = tile_rows(rows);
+  const int64_t tiles = static_cast<int64_t>(p->batch) * p->kv_heads * ((rows + per - 1) / per);
+  const int64_t parts = std::max<int64_t>(1, 512 / std::max<int64_t>(1, tiles));
+  const int64_t part = (std::max<int64_t>(p->max_seqlen, 1) + parts * 64 - 1) / (parts * 64) * 64;
+  return static_cast<int>(std::max<int64_t>(part, per_row));
+}
+
+static int partition_of(const hexkv_attend_params *p) {
+  return use_tiles(p) ? tile_partition(p) : choose_partition(p);
+}
+
 // Partitions per (row, head group) the workspace holds: from the work list
 // when there is one, else from the partition size and max_seqlen.
 static int64_t max_parts_of(const hexkv_attend_params *p, int part) {
@@ -1649,6 +1662,14 @@ static bool use_mfma(const hexkv_attend_params *p, int G) {
 enum LaunchKind { kLaunchValu = 0, kLaunchMfma = 1, kLaunchFt = 2 };
 
 template <typename T, int D, int G>
+static void launch_combine(const AttendArgs &a, hipStream_t s) {
+  const dim3 cgrid(a.q_heads, a.rows);
+  constexpr int SL = kAttThreads / D >= 1 ? kAttThreads / D : 1;
+  if (a.max_parts <= 8 * SL) combine_kernel<T, D, G, 8><<<cgrid, kAttThreads, 0, s>>>(a);
+  else combine_kernel<T, D, G, 32><<<cgrid, kAttThreads, 0, s>>>(a);
+}
+
+template <typename T, int D, int G>
 static void launch(const AttendArgs &a, dim3 grid, int kind, hipStream_t s) {
   if (kind == kLaunchFt) {
     attend_valu_kernel<T, D, G, slots<T, D, G>(), true, true><<<grid, kAttThreads, 0, s>>>(a);
@@ -1658,12 +1679,7 @@ static void launch(const AttendArgs &a, dim3 grid, int kind, hipStream_t s) {
   } else {
     attend_valu_kernel<T, D, G, slots<T, D, G>()><<<grid, kAttThreads, 0, s>>>(a);
   }
-  if (a.max_parts > 1 && !a.seg_count) {
-    const dim3 cgrid(a.q_heads, a.rows);
-    constexpr int SL = kAttThreads / D >= 1 ? kAttThreads / D : 1;
-    if (a.max_parts <= 8 * SL) combine_kernel<T, D, G, 8><<<cgrid, kAttThreads, 0, s>>>(a);
-    else combine_kernel<T, D, G, 32><<<cgrid, kAttThreads, 0, s>>>(a);
-  }
+  if (a.max_parts > 1 && !a.seg_count) launch_combine<T, D, G>(a, s);
 }
 
 // The row-block kernel (head_dim 128, 16-bit): GQ query heads per KV head,
@@ -2032,7 +2048,7 @@ extern "C" size_t hexkv_attend_workspace_bytes(const hexkv_attend_params *p) {
   if (!p || p->q_heads < 1 || p->kv_heads < 1 || p->q_heads % p->kv_heads || p->q_len < 1 ||
       p->batch < 0 || p->max_seqlen < 0)
     return 0;
-  return workspace_bytes(p, choose_partition(p));
+  return workspace_bytes(p, partition_of(p));
 }
 
 extern "C" int hexkv_attend_kernel(const hexkv_attend_params *p) {
@@ -2048,13 +2064,55 @@ extern "C" int hexkv_attend_kernel(const hexkv_attend_params *p) {
 
 namespace hexkv {
 
+// The query-tile kernel on the call `a` describes, and the merge of its
+// partitions when the keys are split.
+static int run_tiles(const hexkv_attend_params *p, const AttendArgs &a, hipStream_t s, const char *what) {
+  TileArgs t{};
+  t.q = a.q;
+  t.q_bs = a.q_bs;
+  t.q_rs = a.q_rs;
+  t.cache = a.cache;
+  t.c_bs = a.c_bs;
+  t.c_ps = a.c_ps;
+  t.c_kv = a.c_kv;
+  t.out = a.out;
+  t.o_bs = a.o_bs;
+  t.o_rs = a.o_rs;
+  t.seqlens = a.seqlens;
+  t.bias = a.bias;
+  t.q_len = a.q_len;
+  t.causal = a.causal;
+  t.q_heads = a.q_heads;
+  t.kv_heads = a.kv_heads;
+  t.group = a.group;
+  t.part = a.part;
+  t.max_parts = a.max_parts;
+  t.max_seqlen = a.max_seqlen;
+  t.scale_log2 = a.scale_log2;
+  t.ws_o = a.ws_o;
+  t.ws_ml = a.ws_ml;
+  t.status = a.status;
+  int rc = launch_tiles(t, p->dtype, p->head_dim, p->batch, s, what);
+  if (rc == HEXKV_OK) rc = check_launch(what);
+  if (rc != HEXKV_OK || a.max_parts <= 1) return rc;
+  // (The merge reads no head group without a work list.)
+  if (p->dtype == HEXKV_BF16) {
+    if (p->head_dim == 128) launch_combine<__bf16, 128, 1>(a, s);
+    else launch_combine<__bf16, 64, 1>(a, s);
+  } else {
+    if (p->head_dim == 128) launch_combine<_Float16, 128, 1>(a, s);
+    else launch_combine<_Float16, 64, 1>(a, s);
+  }
+  return check_launch(what);
+}
+
 // The launch behind hexkv_attend and hexkv_attend_noalloc: validated
 // parameters, a workspace of ws_bytes bytes (device memory), one stream.
 static int attend_launch(const hexkv_attend_params *p, void *workspace, size_t ws_bytes,
                          hexkv_stream_t stream, const char *what) {
   int rc = validate(p);
   if (rc != HEXKV_OK || p->batch == 0) return rc;
-  const int part = choose_partition(p);
+  const int part = partition_of(p);
   const int G = kernel_group(p->q_heads / p->kv_heads);
   const int64_t max_parts = max_parts_of(p, part);
   const size_t need = workspace_bytes(p, part);
@@ -2124,6 +2182,8 @@ static int attend_launch(const hexkv_attend_params *p, void *workspace, size_t w
   if ((a.seqlens || a.items) && (rc = status_word(stream, &a.status, what)) != HEXKV_OK)
     return rc;
 
+  if (use_tiles(p)) return run_tiles(p, a, static_cast<hipStream_t>(stream), what);
+
   dim3 grid;
   if (a.items) {
     grid = dim3(static_cast<unsigned>(p->n_work_items));  // one workgroup per item, in list order
@@ -2183,12 +2243,15 @@ extern "C" int hexkv_attend_noalloc(const hexkv_attend_params *p, hexkv_stream_t
   const char *what = "hexkv_attend_noalloc";
   int rc = validate(p);
   if (rc != HEXKV_OK || p->batch == 0) return rc;
-  const size_t need = workspace_bytes(p, choose_partition(p));
-  if (need > HEXKV_NOALLOC_SCRATCH_BYTES)
+  // The limit is the per-row kernels' need, whichever kernel runs (the tile
+  // kernel never needs more), so it does not depend on the kernel choice.
+  const size_t limit_need = workspace_bytes(p, choose_partition(p));
+  if (limit_need > HEXKV_NOALLOC_SCRATCH_BYTES)
     return fail(HEXKV_EWORKSPACE,
                 "%s: this call needs %zu bytes of split-K workspace, above the %u-byte static scratch "
                 "(use hexkv_attend with a workspace, or fewer rows / a shorter max_seqlen)",
-                what, need, static_cast<unsigned>(HEXKV_NOALLOC_SCRATCH_BYTES));
+                what, limit_need, static_cast<unsigned>(HEXKV_NOALLOC_SCRATCH_BYTES));
+  const size_t need = workspace_bytes(p, partition_of(p));
   void *ws = nullptr;
   if (need > 0 && (rc = scratch_address(stream, &ws, what)) != HEXKV_OK) return rc;
   return attend_launch(p, ws, need, stream, what);

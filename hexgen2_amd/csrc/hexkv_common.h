@@ -237,4 +237,18 @@ struct Elem<float> {
   __device__ __forceinline__ static float from_float(float f) { return f; }
 };
 
+// Four consecutive outputs at p, one vector store when p is aligned for it
+// (output rows may have any element stride).
+template <typename T>
+__device__ __forceinline__ void store4(T *p, f32x4 v) {
+  if ((reinterpret_cast<uintptr_t>(p) & (4 * sizeof(T) - 1)) == 0) {
+    typedef T t4 __attribute__((ext_vector_type(4)));
+    *reinterpret_cast<t4 *>(p) = t4{Elem<T>::from_float(v[0]), Elem<T>::from_float(v[1]),
+                                    Elem<T>::from_float(v[2]), Elem<T>::from_float(v[3])};
+  } else {
+#pragma unroll
+    for (int k = 0; k < 4; ++k) p[k] = Elem<T>::from_float(v[k]);
+  }
+}
+
 }  // namespace hexkv
