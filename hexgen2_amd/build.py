@@ -26,7 +26,8 @@ HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")
 DEVICE_FLAGS = ["-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops"]
 COMMON = ["-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", f"-I{INCLUDE}", f"-I{CSRC}",
           "-Wall", "-Wno-unused-function"]
-SOURCES = ["hexkv_status.cpp", "hexkv_copy.hip", "hexkv_attend.hip", "hexkv_prefill.hip", "hexkv_blocks.hip", "hexkv_ipc.cpp"]
+SOURCES = ["hexkv_status.cpp", "hexkv_copy.hip", "hexkv_attend.hip", "hexkv_prefill.hip", "hexkv_blocks.hip",
+           "hexkv_layer.hip", "hexkv_ipc.cpp"]
 # Register, LDS and occupancy figures of the attention kernels, from the
 # compiler's resource remarks: the work-list planner sizes row-block lists
 # for the workgroups a CU holds at once (tests/test_kernel_resources.py).

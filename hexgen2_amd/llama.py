@@ -9,7 +9,9 @@ calls are exactly the reference's: ``_update_kv_cache`` then
 ``FlashCrossAttention`` (mha.py:565-569), or the fused HIP append+attend;
 with ``fused_ft_kernel`` the decode steps call
 ``_apply_rotary_single_query_attention`` on unrotated q/k (mha.py:553-571).
-Dense projections use torch (hipBLASLt); every KV byte moves through hexkv.
+Dense projections use torch (hipBLASLt), with q/k/v and gate/up each one
+product; the steps between them are one hexkv launch each (residual sum and
+RMSNorm, head split and rotary, SwiGLU), and every KV byte moves through hexkv.
 """
 from __future__ import annotations
 
@@ -20,6 +22,7 @@ from pathlib import Path
 import torch
 import torch.nn.functional as F
 
+from . import ops
 from .mha import FlashCrossAttention, _apply_rotary_single_query_attention, _update_kv_cache, update_and_attend
 
 
@@ -62,14 +65,10 @@ def read_config(model_dir) -> dict:
 
 
 def rms_norm(x: torch.Tensor, weight: torch.Tensor, eps: float) -> torch.Tensor:
-    """rms_norm.py:13-15: normalise in fp32, cast back, scale."""
+    """rms_norm.py:13-15: normalise in fp32, cast back, scale: the plain form
+    of what ``ops.add_rms_norm`` computes in one launch."""
     normalized = x.float() * torch.rsqrt(x.float().square().mean(-1, keepdim=True) + eps)
     return normalized.to(x.dtype) * weight
-
-
-def _rotate_half(x: torch.Tensor) -> torch.Tensor:
-    half = x.shape[-1] // 2
-    return torch.cat((-x[..., half:], x[..., :half]), dim=-1)
 
 
 class LlamaHost:
@@ -81,16 +80,18 @@ class LlamaHost:
         self.device, self.dtype = torch.device(device), dtype
         w = {k: v.to(device=self.device, dtype=dtype) for k, v in weights.items()}
         self.embed = w["model.embed_tokens.weight"]
-        self.norm = w["model.norm.weight"]
+        self.norm = w["model.norm.weight"].contiguous()
         self.lm_head = w["model.embed_tokens.weight"] if shape.tie_word_embeddings else w["lm_head.weight"]
         self.layers = []
         for i in range(shape.num_hidden_layers):
             p = f"model.layers.{i}."
+            # projections of one input are one matrix each, laid out once
             self.layers.append({
-                "ln1": w[p + "input_layernorm.weight"], "ln2": w[p + "post_attention_layernorm.weight"],
-                "wq": w[p + "self_attn.q_proj.weight"], "wk": w[p + "self_attn.k_proj.weight"],
-                "wv": w[p + "self_attn.v_proj.weight"], "wo": w[p + "self_attn.o_proj.weight"],
-                "gate": w[p + "mlp.gate_proj.weight"], "up": w[p + "mlp.up_proj.weight"],
+                "ln1": w[p + "input_layernorm.weight"].contiguous(),
+                "ln2": w[p + "post_attention_layernorm.weight"].contiguous(),
+                "wqkv": torch.cat([w.pop(p + f"self_attn.{n}_proj.weight") for n in "qkv"]),
+                "wo": w[p + "self_attn.o_proj.weight"],
+                "gate_up": torch.cat([w.pop(p + f"mlp.{n}_proj.weight") for n in ("gate", "up")]),
                 "down": w[p + "mlp.down_proj.weight"],
             })
         d = shape.head_dim
@@ -114,24 +115,6 @@ class LlamaHost:
             state.update(values)
         return cls(shape, state, device, dtype)
 
-    def _rope(self, x: torch.Tensor, offset: int, positions=None) -> torch.Tensor:
-        """Rotary (GPT-NeoX halves) of ``x [B, S, H, D]`` at positions
-        ``offset + s``, or for one new token per sequence (S == 1) at each
-        sequence's own ``positions[b]`` (a ragged decode batch)."""
-        seqlen = x.shape[1]
-        if positions is not None:
-            freqs = positions.to(torch.float32)[:, None] * self.inv_freq[None, :]  # [B, D/2]
-            emb = torch.cat((freqs, freqs), dim=-1)
-            cos = emb.cos().to(x.dtype)[:, None, None, :]
-            sin = emb.sin().to(x.dtype)[:, None, None, :]
-            return x * cos + _rotate_half(x) * sin
-        pos = torch.arange(offset, offset + seqlen, device=self.device, dtype=torch.float32)
-        freqs = torch.outer(pos, self.inv_freq)
-        emb = torch.cat((freqs, freqs), dim=-1)
-        cos = emb.cos().to(x.dtype)[None, :, None, :]
-        sin = emb.sin().to(x.dtype)[None, :, None, :]
-        return x * cos + _rotate_half(x) * sin
-
     @torch.inference_mode()
     def forward(self, input_ids: torch.Tensor, inference_params, last_token_only: bool = True,
                 fused_append: bool = False) -> torch.Tensor:
@@ -144,29 +127,29 @@ class LlamaHost:
         positions = None
         if inference_params.lengths_per_sample is not None and seqlen == 1 and offset > 0:
             b0 = inference_params.batch_size_offset
-            positions = inference_params.lengths_per_sample[b0:b0 + batch]
+            positions = inference_params.lengths_per_sample[b0:b0 + batch].to(torch.int32).contiguous()
+        heads, kv_heads = s.num_attention_heads, s.num_key_value_heads
         h = F.embedding(input_ids, self.embed)
+        y = None  # the block output still to be added to h
         for i, layer in enumerate(self.layers):
-            x = rms_norm(h, layer["ln1"], s.rms_norm_eps)
-            q = (x @ layer["wq"].T).view(batch, seqlen, s.num_attention_heads, d)
-            k = (x @ layer["wk"].T).view(batch, seqlen, s.num_key_value_heads, d)
-            v = (x @ layer["wv"].T).view(batch, seqlen, s.num_key_value_heads, d)
+            x = ops.add_rms_norm(h, y, layer["ln1"], s.rms_norm_eps)
+            qkv = F.linear(x, layer["wqkv"])
             if inference_params.fused_ft_kernel and offset > 0:
                 # FT decode (mha.py:553-571): rotary, append and attention in one call
-                context = _apply_rotary_single_query_attention(q, inference_params, i, d, s.rope_theta,
-                                                               kv=torch.stack((k, v), dim=2))
+                q = qkv[..., :heads * d].view(batch, seqlen, heads, d)
+                kv = qkv[..., heads * d:].view(batch, seqlen, 2, kv_heads, d)
+                context = _apply_rotary_single_query_attention(q, inference_params, i, d, s.rope_theta, kv=kv)
             else:
-                q, k = self._rope(q, offset, positions), self._rope(k, offset, positions)
-                kv = torch.stack((k, v), dim=2)  # [B, S, 2, Hkv, D]
+                q, kv = ops.rope_split(qkv, heads, kv_heads, d, self.inv_freq, offset, positions)
                 if fused_append and offset > 0 and seqlen == 1 and i in inference_params.key_value_memory_dict:
                     context = update_and_attend(q, kv, inference_params, i, self.scale)
                 else:
                     kv_view = _update_kv_cache(kv, inference_params, i)
                     # prompt (offset 0): causal; decode: causal=False (mha.py:566-569)
                     context = self.attn(q, kv_view, causal=None if offset == 0 else False)
-            h = h + context.reshape(batch, seqlen, -1) @ layer["wo"].T
-            x = rms_norm(h, layer["ln2"], s.rms_norm_eps)
-            h = h + (F.silu(x @ layer["gate"].T) * (x @ layer["up"].T)) @ layer["down"].T
+            y = F.linear(context.reshape(batch, seqlen, -1), layer["wo"])
+            x = ops.add_rms_norm(h, y, layer["ln2"], s.rms_norm_eps)
+            y = F.linear(ops.silu_mul(F.linear(x, layer["gate_up"])), layer["down"])
         if last_token_only:
-            h = h[:, -1]
-        return rms_norm(h, self.norm, s.rms_norm_eps) @ self.lm_head.T
+            h, y = h[:, -1], None if y is None else y[:, -1]
+        return F.linear(ops.add_rms_norm(h, y, self.norm, s.rms_norm_eps, keep_sum=False), self.lm_head)

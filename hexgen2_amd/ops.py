@@ -633,6 +633,91 @@ def ft_attend(q: torch.Tensor, k_new: torch.Tensor, v_new: torch.Tensor, k_cache
     return out
 
 
+def add_rms_norm(h: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tensor, eps: float,
+                 keep_sum: bool = True) -> torch.Tensor:
+    """``rms_norm(h + y) * weight`` over the last dim, one launch, contiguous
+    (rms_norm.py:13-15 after block.py:112-175's residual sum).  ``y`` None:
+    no sum.  With ``keep_sum`` the sum replaces ``h`` in place.  ``h`` and
+    ``y`` are ``[..., hidden]`` whose rows lie at one stride."""
+    _require_device(h, weight)
+    hidden = h.shape[-1]
+    rows = h.numel() // hidden if hidden else 0
+    if h.dtype not in _DTYPES or weight.dtype != h.dtype or weight.device != h.device:
+        raise ValueError("h and weight must share one of float16, bfloat16, float32 and a device")
+    if weight.shape != (hidden,) or not weight.is_contiguous():
+        raise ValueError(f"weight must be contiguous [{hidden}], got {tuple(weight.shape)}")
+    y_ptr, y_stride = None, 0
+    if y is not None:
+        _require_device(y)
+        if y.shape != h.shape or y.dtype != h.dtype or y.device != h.device:
+            raise ValueError("h and y must share shape, dtype and device")
+        y_ptr, y_stride = y.data_ptr(), _row_stride(y, "y")
+    h_stride = _row_stride(h, "h")
+    out = torch.empty(h.shape, dtype=h.dtype, device=h.device)
+    kept = h.data_ptr() if keep_sum and y is not None else None
+    rc = _lib.load().hexkv_add_rms_norm(h.data_ptr(), h_stride, y_ptr, y_stride, kept, h_stride, weight.data_ptr(),
+                                        out.data_ptr(), rows, hidden, eps, _DTYPES[h.dtype], _stream(h))
+    _lib.check(rc, "hexkv_add_rms_norm")
+    return out
+
+
+def _row_stride(t: torch.Tensor, name: str) -> int:
+    """Elements between consecutive rows (last dim) of ``t``, whose outer
+    dims must fold into one."""
+    if t.is_contiguous():
+        return t.shape[-1]
+    if t.stride(-1) != 1 or t.dim() != 2:
+        raise ValueError(f"{name} rows must be contiguous and lie at one stride")
+    return t.stride(0)
+
+
+def rope_split(qkv: torch.Tensor, q_heads: int, kv_heads: int, head_dim: int, inv_freq: torch.Tensor,
+               offset: int = 0, positions: Optional[torch.Tensor] = None):
+    """Split ``qkv [B, S, (q_heads + 2 kv_heads) * D]`` (contiguous) into
+    ``q [B, S, q_heads, D]`` and ``kv [B, S, 2, kv_heads, D]``, q and k
+    rotated (GPT-NeoX halves) by ``position * inv_freq``: position
+    ``offset + s``, or ``positions[b]`` (device int32) for every token of
+    sequence b.  One launch; sines, cosines and the turn in fp32."""
+    _require_device(qkv, inv_freq)
+    if qkv.dim() != 3 or qkv.shape[2] != (q_heads + 2 * kv_heads) * head_dim or not qkv.is_contiguous():
+        raise ValueError(f"qkv must be contiguous [B, S, {(q_heads + 2 * kv_heads) * head_dim}], "
+                         f"got {tuple(qkv.shape)}")
+    if qkv.dtype not in _DTYPES:
+        raise ValueError("qkv must be one of float16, bfloat16, float32")
+    if inv_freq.dtype != torch.float32 or inv_freq.shape != (head_dim // 2,) or not inv_freq.is_contiguous() \
+            or inv_freq.device != qkv.device:
+        raise ValueError("inv_freq must be contiguous float32 [head_dim / 2] on qkv's device")
+    batch, seqlen = qkv.shape[:2]
+    pos_ptr = None
+    if positions is not None:
+        _require_device(positions)
+        if positions.dtype != torch.int32 or positions.numel() < batch or not positions.is_contiguous():
+            raise ValueError("positions must be a contiguous int32 device tensor with one entry per sequence")
+        pos_ptr = positions.data_ptr()
+    q = torch.empty((batch, seqlen, q_heads, head_dim), dtype=qkv.dtype, device=qkv.device)
+    kv = torch.empty((batch, seqlen, 2, kv_heads, head_dim), dtype=qkv.dtype, device=qkv.device)
+    rc = _lib.load().hexkv_rope_split(qkv.data_ptr(), qkv.shape[2], inv_freq.data_ptr(), pos_ptr, int(offset),
+                                      q.data_ptr(), kv.data_ptr(), batch * seqlen, max(seqlen, 1), q_heads, kv_heads,
+                                      head_dim, _DTYPES[qkv.dtype], _stream(qkv))
+    _lib.check(rc, "hexkv_rope_split")
+    return q, kv
+
+
+def silu_mul(gate_up: torch.Tensor) -> torch.Tensor:
+    """``silu(gate) * up`` of ``gate_up [..., 2 * width]`` (contiguous, gate
+    first), one launch: the SwiGLU of mlp.py:63-87."""
+    _require_device(gate_up)
+    if gate_up.dtype not in _DTYPES or gate_up.shape[-1] % 2 or not gate_up.is_contiguous():
+        raise ValueError(f"gate_up must be contiguous [..., 2 * width] in float16, bfloat16 or float32, "
+                         f"got {tuple(gate_up.shape)} {gate_up.dtype}")
+    width = gate_up.shape[-1] // 2
+    out = torch.empty((*gate_up.shape[:-1], width), dtype=gate_up.dtype, device=gate_up.device)
+    rc = _lib.load().hexkv_silu_mul(gate_up.data_ptr(), out.data_ptr(), out.numel() // max(width, 1), width,
+                                    _DTYPES[gate_up.dtype], _stream(gate_up))
+    _lib.check(rc, "hexkv_silu_mul")
+    return out
+
+
 def _tensor_geometry(t: Optional[torch.Tensor]):
     """Everything about a tensor a prebuilt parameter block depends on apart
     from its address: shape, strides (which fix its contiguity), dtype and

@@ -564,6 +564,29 @@ int hexkv_ipc_close(void *base);
 void *hexkv_ipc_dlpack(void *base, uint64_t offset, int ndim, const int64_t *shape,
                        int dtype_code, int dtype_bits, int device_id);
 
+/* ------------------------------------------------- decoder layer steps ---
+ * The steps between a decoder layer's matrix products, one launch each (the
+ * reference runs them as separate tensor operations).  Strides are in
+ * elements, rows of `out`, `q` and `kv` are contiguous, below 2^24 rows. */
+
+/* out[r] = rms_norm(h[r] + y[r]) * weight (rms_norm.py:13-15; the residual
+ * sum of modules/block.py:112-175).  y NULL: no sum.  h_out (may be h, or
+ * NULL) receives the sum rounded to the data type. */
+int hexkv_add_rms_norm(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
+                       int64_t h_out_stride, const void *weight, void *out, int64_t rows, int hidden,
+                       float eps, int dtype, hexkv_stream_t stream);
+
+/* Rows [q heads | k heads | v heads] of head_dim elements (qkv_stride apart)
+ * into q [rows][q_heads][head_dim] and kv [rows][2][kv_heads][head_dim], q
+ * and k rotated (GPT-NeoX halves) by position * inv_freq_dev[j].  Row r is
+ * position r % seqlen + offset, or positions_dev[r / seqlen] when given. */
+int hexkv_rope_split(const void *qkv, int64_t qkv_stride, const float *inv_freq_dev,
+                     const int32_t *positions_dev, int offset, void *q, void *kv, int64_t rows, int seqlen,
+                     int q_heads, int kv_heads, int head_dim, int dtype, hexkv_stream_t stream);
+
+/* out[r][i] = silu(gate_up[r][i]) * gate_up[r][width + i] (mlp.py:63-87). */
+int hexkv_silu_mul(const void *gate_up, void *out, int64_t rows, int width, int dtype, hexkv_stream_t stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1,0 +1,91 @@
+"""The fused decoder-layer steps (residual + RMSNorm, head split + rotary,
+SwiGLU) against 64-bit forms of the same operations, at the edges of their
+vector, register and scalar paths.  Bounds: one rounding to the data type per
+rounding the kernel makes (unit roundoff ``u``), plus a few fp32 roundings."""
+import pytest
+import torch
+
+from hexgen2_amd import ops
+from hexgen2_amd.llama import rms_norm
+
+pytestmark = pytest.mark.gpu
+
+DTYPES = [torch.float16, torch.bfloat16, torch.float32]
+# half a spacing relative to the value: 2^-p for p significant bits (11, 8, 24)
+UNIT = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8, torch.float32: 2.0 ** -24}
+FP32 = 2.0 ** -20  # a sum of squares of up to 2^13 terms in pairwise order, rsqrt, a division
+TINY = 2.0 ** -24  # spacing of the smallest float16 values
+
+
+def _within(got, want, bound):
+    assert torch.isfinite(got.double()).all()
+    assert ((got.double() - want).abs() <= bound).all(), float(((got.double() - want).abs() - bound).max())
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("hidden", [1, 7, 64, 1024, 2048, 2056, 4096, 4104, 8192, 8200, 8201])
+@pytest.mark.parametrize("with_y", [False, True])
+def test_add_rms_norm(dtype, hidden, with_y):
+    torch.manual_seed(hidden)
+    h, y = (torch.randn(2, 3, hidden, device="cuda").to(dtype) for _ in range(2))
+    w = torch.randn(hidden, device="cuda").to(dtype)
+    want_h = h + y if with_y else h.clone()
+    kept = h.clone()
+    out = ops.add_rms_norm(kept, y if with_y else None, w, 1e-5)
+    assert torch.equal(kept, want_h)
+    x = want_h.double()
+    want = x * torch.rsqrt(x.square().mean(-1, keepdim=True) + 1e-5) * w.double()
+    bound = (2.1 * UNIT[dtype] + FP32) * want.abs() + TINY * (1 + w.double().abs())
+    _within(out, want, bound)
+    _within(rms_norm(want_h, w, 1e-5), want, bound)
+    # the last token of each sequence: rows 3 * hidden apart, h left alone
+    last = ops.add_rms_norm(h[:, -1], y[:, -1] if with_y else None, w, 1e-5, keep_sum=False)
+    assert torch.equal(last, out[:, -1])
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("heads,kv_heads,dim", [(4, 4, 16), (32, 4, 64), (8, 1, 128), (32, 32, 128), (3, 1, 6), (5, 5, 20)])
+@pytest.mark.parametrize("ragged", [False, True])
+def test_rope_split(dtype, heads, kv_heads, dim, ragged):
+    torch.manual_seed(dim)
+    batch, seqlen, offset = (3, 1, 0) if ragged else (2, 9, 4091)
+    qkv = torch.randn(batch, seqlen, (heads + 2 * kv_heads) * dim, device="cuda").to(dtype)
+    inv = 1.0 / (10000.0 ** (torch.arange(0, dim, 2, device="cuda", dtype=torch.float32) / dim))
+    at = torch.tensor([0, 17, 8191], dtype=torch.int32, device="cuda") if ragged else None
+    q, kv = ops.rope_split(qkv, heads, kv_heads, dim, inv, offset, at)
+    qk, v = qkv[..., :(heads + kv_heads) * dim], qkv[..., (heads + kv_heads) * dim:]
+    pos = at.float()[:, None] if ragged else (offset + torch.arange(seqlen, device="cuda").float())[None].expand(batch, -1)
+    angle = (pos[..., None] * inv).double()[:, :, None]  # the fp32 product, as the kernel forms it
+    x = qk.double().view(batch, seqlen, heads + kv_heads, dim)
+    a, b = x[..., :dim // 2], x[..., dim // 2:]
+    want = torch.cat((a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin()), -1)
+    got = torch.cat((q, kv[:, :, 0]), 2)
+    size = (a.abs() + b.abs()).repeat(1, 1, 1, 2)
+    _within(got, want, UNIT[dtype] * 1.01 * want.abs() + FP32 * size + TINY)
+    assert torch.equal(kv[:, :, 1].reshape(v.shape), v)
+
+
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("width", [1, 7, 255, 256, 2048, 2056, 5632])
+def test_silu_mul(dtype, width):
+    torch.manual_seed(width)
+    gate_up = (4 * torch.randn(3, 2, 2 * width, device="cuda")).to(dtype)
+    g, u = gate_up.double().chunk(2, -1)
+    want = g * torch.sigmoid(g) * u
+    _within(ops.silu_mul(gate_up), want, (UNIT[dtype] * 1.01 + FP32) * want.abs() + TINY)
+
+
+def test_layer_steps_refuse_what_they_cannot_address():
+    x = torch.zeros(2, 3, 8, device="cuda", dtype=torch.float16)
+    w = torch.zeros(8, device="cuda", dtype=torch.float16)
+    with pytest.raises(ValueError):
+        ops.add_rms_norm(x, None, w[:4], 1e-5)
+    with pytest.raises(ValueError):
+        ops.add_rms_norm(x.transpose(0, 1), None, w, 1e-5)
+    with pytest.raises(ValueError):
+        ops.add_rms_norm(x, x.float(), w, 1e-5)
+    with pytest.raises(ValueError):
+        ops.silu_mul(x[..., :6])
+    with pytest.raises(ValueError):
+        ops.rope_split(x, 2, 1, 2, torch.zeros(2, device="cuda"))
+    assert ops.silu_mul(x[:0]).shape == (0, 3, 4)
