@@ -23,7 +23,9 @@ EXPORTS = ("hexkv_version", "hexkv_last_error", "hexkv_pack", "hexkv_unpack", "h
            "hexkv_head_concat", "hexkv_ipc_export", "hexkv_ipc_open", "hexkv_ipc_close",
            "hexkv_ipc_dlpack", "hexkv_ft_store", "hexkv_ft_attend_workspace_bytes", "hexkv_ft_attend",
            "hexkv_attend_noalloc", "hexkv_attend_plan", "hexkv_attend_plan_chunk", "hexkv_attend_plan_kernel",
-           "hexkv_device_status", "hexkv_device_xcds", "hexkv_add_rms_norm", "hexkv_rope_split", "hexkv_silu_mul")
+           "hexkv_device_status", "hexkv_device_xcds", "hexkv_add_rms_norm", "hexkv_rope_split", "hexkv_silu_mul",
+           "hexkv_attend_layers", "hexkv_attend_layers_workspace_bytes", "hexkv_attend_layers_independent",
+           "hexkv_attend_plan_layers")
 NOALLOC_SCRATCH_BYTES = 32 << 20
 # Arrival counters at the front of every attention workspace (zero them once).
 ATTEND_COUNTER_BYTES = 256 << 10
@@ -50,6 +52,12 @@ class AttendParams(ctypes.Structure):
         ("n_work_items", ctypes.c_int32), ("work_max_parts", ctypes.c_int32),
         ("work_xcds", ctypes.c_int32), ("lengths_out_dev", ctypes.c_void_p),
     ]
+
+
+class AttendLayer(ctypes.Structure):
+    """Mirror of ``hexkv_attend_layer``."""
+    _fields_ = [("q", ctypes.c_void_p), ("cache", ctypes.c_void_p), ("out", ctypes.c_void_p),
+                ("kv_new", ctypes.c_void_p)]
 
 
 class WorkItem(ctypes.Structure):
@@ -123,6 +131,11 @@ def load() -> ctypes.CDLL:
     lib.hexkv_attend_kernel.argtypes = [ctypes.POINTER(AttendParams)]
     lib.hexkv_attend.restype = ci
     lib.hexkv_attend.argtypes = [ctypes.POINTER(AttendParams), vp, ctypes.c_size_t, vp]
+    layers = ctypes.POINTER(AttendLayer)
+    lib.hexkv_attend_layers_workspace_bytes.restype = ctypes.c_size_t
+    lib.hexkv_attend_layers_workspace_bytes.argtypes = [ctypes.POINTER(AttendParams), layers, ci]
+    lib.hexkv_attend_layers.restype = ci
+    lib.hexkv_attend_layers.argtypes = [ctypes.POINTER(AttendParams), layers, vp, ci, vp, ctypes.c_size_t, vp]
     i32p = ctypes.POINTER(ctypes.c_int32)
     lib.hexkv_attend_plan.restype = ci
     lib.hexkv_attend_plan.argtypes = [ctypes.POINTER(AttendParams), vp, vp, ctypes.c_int32, vp, ctypes.c_int32,
@@ -131,6 +144,10 @@ def load() -> ctypes.CDLL:
     lib.hexkv_attend_plan_chunk.argtypes = [ctypes.POINTER(AttendParams), vp, i32p]
     lib.hexkv_attend_plan_kernel.restype = ci
     lib.hexkv_attend_plan_kernel.argtypes = [ctypes.POINTER(AttendParams), vp, i32p]
+    lib.hexkv_attend_plan_layers.restype = ci
+    lib.hexkv_attend_plan_layers.argtypes = [ctypes.POINTER(AttendParams), vp, ci, i32p, i32p]
+    lib.hexkv_attend_layers_independent.restype = ci
+    lib.hexkv_attend_layers_independent.argtypes = [ctypes.POINTER(AttendParams), layers, ci]
     lib.hexkv_attend_noalloc.restype = ci
     lib.hexkv_attend_noalloc.argtypes = [ctypes.POINTER(AttendParams), vp]
     blocks = ctypes.POINTER(Block)

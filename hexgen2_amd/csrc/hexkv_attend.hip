@@ -116,6 +116,10 @@ struct AttendArgs {
   // own XCD within its group of n_xcd (see begin_work).
   int32_t xcd_remap;
   int32_t *lengths_out;  // work lists with kv_new: row b's new length, or nullptr
+  // Several independent layers in one launch (work lists; grid y = layer):
+  // their tensors, and the partials of layer l l * layer_slots slots on.
+  const hexkv_attend_layer *layers;
+  int64_t layer_slots;
   unsigned int *status;  // HEXKV_STATUS_* word of this device, or nullptr
   // FasterTransformer cache layouts (hexkv_ft_attend only): K is
   // [batch][kv_heads][D / pack][capacity][pack] (one 16-byte chunk of D per
@@ -131,6 +135,33 @@ struct AttendArgs {
   int32_t rot_neox;     // 1: pairs (i, i + rot_dim / 2); 0: pairs (2i, 2i + 1)
   double rot_log2_base;  // log2 of the rotary base
 };
+
+// This workgroup's arguments: those of its layer when the launch holds
+// several (the last layer records the new lengths).  A layer's own launch
+// costs its ramp and its tail, ~4 us, on work of the same order: the
+// Llama-2-70B TP-8 share's 16 layers (43 MB each) took 196 us as 16 launches
+// and take 133 us as one.
+// A launch of one layer has its own kernels: testing for the table at run
+// time cost it ~0.7 us.
+template <bool LAYERS>
+__device__ __forceinline__ AttendArgs layer_args(const AttendArgs &args, int head_dim) {
+  AttendArgs a = args;
+  if constexpr (LAYERS) {
+    const int64_t l = blockIdx.y;
+    const hexkv_attend_layer t = args.layers[l];
+    a.q = t.q;
+    a.cache = t.cache;
+    a.out = t.out;
+    a.kv_new = t.kv_new;
+    if (args.seg_count) {
+      a.ws_o += l * args.layer_slots * head_dim;
+      a.ws_ml += l * args.layer_slots * 2;
+      a.seg_count += l * args.rows * args.n_groups;
+    }
+    if (blockIdx.y + 1 != gridDim.y) a.lengths_out = nullptr;
+  }
+  return a;
+}
 
 // Number of keys query row (b, t) attends to; *pos_new = cache position of the
 // fused-append row (or -1).
@@ -181,7 +212,7 @@ __device__ __forceinline__ bool begin_work(const AttendArgs &a, Work &w) {
     // reports it.  (One device-scope atomic per workgroup, as every split
     // item once did at its merge, cost ~1 us per call at the Llama-2-70B
     // TP-8 share whenever the rotation was not 0.)
-    if (a.seg_count && a.n_xcd > 0 && blockIdx.x == 0 && threadIdx.x == 0 &&
+    if (a.seg_count && a.n_xcd > 0 && blockIdx.x == 0 && blockIdx.y == 0 && threadIdx.x == 0 &&
         static_cast<unsigned>(xcd_id()) % a.n_xcd != 0)
       raise_status(a.status, HEXKV_STATUS_DISPATCH);
     const hexkv_work_item it = a.items[idx];
@@ -480,8 +511,8 @@ __device__ __forceinline__ void ft_prologue(const AttendArgs &a, const Work &w, 
 
 // ------------------------------------------------------------- VALU path ---
 
-template <typename T, int D, int G, int U, bool PF = true, bool FT = false>
-__global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendArgs a) {
+template <typename T, int D, int G, int U, bool PF = true, bool FT = false, bool LAYERS = false>
+__global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendArgs args) {
   using E = Elem<T>;
   using L = Lanes<T, D>;
   constexpr int VEC = L::VEC, NV = L::NV, EPL = L::EPL, LPP = L::LPP, GPW = L::GPW, NG = L::NG;
@@ -493,6 +524,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
   // one padded row per position.
   constexpr int KT_PITCH = D / VEC * 16 + 16;
   __shared__ __attribute__((aligned(16))) char s_kt[FT ? 2 * STEP * KT_PITCH : 16];
+  const AttendArgs a = layer_args<LAYERS>(args, D);
   Work w;
   if (!begin_work<T, D, G>(a, w)) return;
 
@@ -830,8 +862,8 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
 // its head's GQ query heads; the slots of a head are merged through LDS at
 // the end (finish_work over NG / HB slots), and a split segment
 // (row, head block) merges XCD-locally like the other kernels'.
-template <typename T, int D, int GQ, int HB, int U>
-__global__ __launch_bounds__(kAttThreads) void attend_rows_kernel(const AttendArgs a) {
+template <typename T, int D, int GQ, int HB, int U, bool LAYERS = false>
+__global__ __launch_bounds__(kAttThreads) void attend_rows_kernel(const AttendArgs args) {
   using E = Elem<T>;
   using L = Lanes<T, D>;
   constexpr int VEC = L::VEC, NV = L::NV, EPL = L::EPL, LPP = L::LPP, GPW = L::GPW, NG = L::NG;
@@ -839,6 +871,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_rows_kernel(const AttendAr
   static_assert(NG % HB == 0, "the head block divides the lane groups");
   __shared__ __attribute__((aligned(16))) float s_acc[PS][QH][D];
   __shared__ float s_m[PS][QH], s_l[PS][QH];
+  const AttendArgs a = layer_args<LAYERS>(args, D);
   Work w;
   if (!begin_work<T, D, QH>(a, w)) return;
 
@@ -1097,8 +1130,8 @@ struct Mfma<_Float16> {
 // Three waves per SIMD (at most 168 registers per lane): measured faster than
 // two (more registers, accumulators in AGPRs) and than four on the
 // Llama-2-70B TP-8 share (16.8 vs 19.7 and 18.4 us per layer).
-template <typename T, int D, int G>
-__global__ __launch_bounds__(kAttThreads, 3) void attend_mfma_kernel(const AttendArgs a) {
+template <typename T, int D, int G, bool LAYERS = false>
+__global__ __launch_bounds__(kAttThreads, 3) void attend_mfma_kernel(const AttendArgs args) {
   static_assert(sizeof(T) == 2 && G <= 16, "MFMA path: 16-bit types, up to 16 heads per group");
   using M = Mfma<T>;
   constexpr int NJ = D / 32;         // score k-steps of 32 elements
@@ -1111,6 +1144,7 @@ __global__ __launch_bounds__(kAttThreads, 3) void attend_mfma_kernel(const Atten
   __shared__ __attribute__((aligned(16))) char s_v[kAttWaves][16 * PITCH];
   __shared__ __attribute__((aligned(16))) float s_acc[kAttWaves][G][D];
   __shared__ float s_m[kAttWaves][G], s_l[kAttWaves][G];
+  const AttendArgs a = layer_args<LAYERS>(args, D);
   Work w;
   if (!begin_work<T, D, G>(a, w)) return;
 
@@ -1671,37 +1705,43 @@ static void launch_combine(const AttendArgs &a, hipStream_t s) {
 
 template <typename T, int D, int G>
 static void launch(const AttendArgs &a, dim3 grid, int kind, hipStream_t s) {
+  constexpr int U = slots<T, D, G>();
   if (kind == kLaunchFt) {
-    attend_valu_kernel<T, D, G, slots<T, D, G>(), true, true><<<grid, kAttThreads, 0, s>>>(a);
-  } else if constexpr (sizeof(T) == 2 && D >= 64) {
-    if (kind == kLaunchMfma) attend_mfma_kernel<T, D, G><<<grid, kAttThreads, 0, s>>>(a);
-    else attend_valu_kernel<T, D, G, slots<T, D, G>()><<<grid, kAttThreads, 0, s>>>(a);
-  } else {
-    attend_valu_kernel<T, D, G, slots<T, D, G>()><<<grid, kAttThreads, 0, s>>>(a);
+    attend_valu_kernel<T, D, G, U, true, true><<<grid, kAttThreads, 0, s>>>(a);
+    if (a.max_parts > 1) launch_combine<T, D, G>(a, s);
+    return;
   }
+  if constexpr (sizeof(T) == 2 && D >= 64) {
+    if (kind == kLaunchMfma) {
+      if (a.layers) attend_mfma_kernel<T, D, G, true><<<grid, kAttThreads, 0, s>>>(a);
+      else attend_mfma_kernel<T, D, G><<<grid, kAttThreads, 0, s>>>(a);
+      if (a.max_parts > 1 && !a.seg_count) launch_combine<T, D, G>(a, s);
+      return;
+    }
+  }
+  if (a.layers) attend_valu_kernel<T, D, G, U, true, false, true><<<grid, kAttThreads, 0, s>>>(a);
+  else attend_valu_kernel<T, D, G, U><<<grid, kAttThreads, 0, s>>>(a);
   if (a.max_parts > 1 && !a.seg_count) launch_combine<T, D, G>(a, s);
 }
 
 // The row-block kernel (head_dim 128, 16-bit): GQ query heads per KV head,
 // HB KV heads per item.
+template <typename T, int GQ, int HB>
+static int launch_rows(const AttendArgs &a, dim3 grid, hipStream_t s) {
+  constexpr int U = slots<T, 128, GQ>();
+  if (a.layers) attend_rows_kernel<T, 128, GQ, HB, U, true><<<grid, kAttThreads, 0, s>>>(a);
+  else attend_rows_kernel<T, 128, GQ, HB, U><<<grid, kAttThreads, 0, s>>>(a);
+  return HEXKV_OK;
+}
+
 template <typename T, int GQ>
 static int dispatch_rows_hb(int HB, const AttendArgs &a, dim3 grid, hipStream_t s) {
   // The head blocks rows_block picks: 2 KV heads for grouped queries; 8, 4
   // or 2 for one query head per KV head.
-  constexpr int U = slots<T, 128, GQ>();
-  if (HB == 2) {
-    attend_rows_kernel<T, 128, GQ, 2, U><<<grid, kAttThreads, 0, s>>>(a);
-    return HEXKV_OK;
-  }
+  if (HB == 2) return launch_rows<T, GQ, 2>(a, grid, s);
   if constexpr (GQ == 1) {
-    if (HB == 4) {
-      attend_rows_kernel<T, 128, GQ, 4, U><<<grid, kAttThreads, 0, s>>>(a);
-      return HEXKV_OK;
-    }
-    if (HB == 8) {
-      attend_rows_kernel<T, 128, GQ, 8, U><<<grid, kAttThreads, 0, s>>>(a);
-      return HEXKV_OK;
-    }
+    if (HB == 4) return launch_rows<T, GQ, 4>(a, grid, s);
+    if (HB == 8) return launch_rows<T, GQ, 8>(a, grid, s);
   }
   return fail(HEXKV_EUNSUPPORTED, "hexkv_attend: head block %d with %d query heads per KV head", HB, GQ);
 }
@@ -1935,6 +1975,72 @@ extern "C" int hexkv_attend_plan_kernel(const hexkv_attend_params *p, const int3
 
 namespace hexkv {
 
+static bool layers_independent(const hexkv_attend_params *p, const hexkv_attend_layer *layers, int n_layers);
+
+// Lists whose layers share launches (hexkv_attend_layers).  Layers below
+// kSharedLayerBytes each: above, a layer keeps the chip busy for so long that
+// its own tail hardly counts (Llama-3-8B, 64 rows, 963 MB a layer: 592 us for
+// four layers sharing, 588 in order; 32 rows, 327 MB: 219 and 221).  Their
+// items fill the chip together, so the chunk follows the launch's positions,
+// about two items per CU over all its layers, and is cut off where items
+// become too large to balance (384 KB a one-head item, 768 KB a row-block
+// one).  Measured per replay on MI355X, this rule's chunk against the
+// one-layer rule's: Llama-2-70B TP-8 share (16 layers of 43 MB) 128.5 us at
+// 768 positions, 135.4 at 384; Llama-2-7B (4 of 122 MB) 79-84 at 128-256
+// against 88.7 at 112; Llama-3-8B with 8 rows (4 of 31 MB) 27.2-29.2 with
+// row blocks at 128-256, 32.7 with one head per item.
+constexpr int64_t kSharedLayerBytes = INT64_C(512) << 20;
+constexpr int64_t kSharedItems = 512;
+
+}  // namespace hexkv
+
+extern "C" int hexkv_attend_plan_layers(const hexkv_attend_params *p, const int32_t *lens, int n_layers,
+                                        int32_t *kernel, int32_t *chunk) {
+  using namespace hexkv;
+  clear_error();
+  const char *what = "hexkv_attend_plan_layers";
+  if (!p || !kernel || !chunk || n_layers < 1) return fail(HEXKV_EINVAL, "%s: null argument or no layer", what);
+  hexkv_attend_params one = *p;
+  one.partition = 0;
+  int rc = hexkv_attend_plan_kernel(&one, lens, &one.kernel);
+  if (rc != HEXKV_OK) return rc;
+  int64_t positions = 0, longest = 0;
+  for (int b = 0; b < p->batch; ++b) {
+    const int64_t len = static_cast<int64_t>(lens[b]) + p->seqlen_bias + (p->kv_new ? 1 : 0);
+    positions += len;
+    longest = std::max(longest, len);
+  }
+  const int64_t row_bytes = 2 * static_cast<int64_t>(p->head_dim) * elem_size(p->dtype);
+  const int64_t bytes = positions * p->kv_heads * row_bytes;
+  const bool shared = n_layers > 1 && p->work_xcds >= 1 && p->work_xcds <= 8 && bytes < kSharedLayerBytes;
+  if (shared && p->kernel == HEXKV_KERNEL_AUTO && rows_block(p) && bytes * n_layers >= (INT64_C(64) << 20))
+    one.kernel = HEXKV_KERNEL_ROWS;
+  one.partition = p->partition;
+  const int c = plan_request(&one, lens, what);
+  if (c < 0) return c;
+  *kernel = one.kernel;
+  *chunk = c;
+  if (!shared || p->partition > 0) return HEXKV_OK;
+  const bool rows = one.kernel == HEXKV_KERNEL_ROWS;
+  const int64_t grain = rows ? 16 : 64;
+  const auto up = [grain](int64_t v) { return (v + grain - 1) / grain * grain; };
+  const int64_t groups = p->q_heads / segment_heads(&one);
+  const int64_t most = rows ? (INT64_C(768) << 10) / (row_bytes * rows_block(p)) : (INT64_C(384) << 10) / row_bytes;
+  const int64_t fewest = std::max<int64_t>(64, (longest + kMergeMaxParts - 1) / kMergeMaxParts);
+  *chunk = static_cast<int32_t>(up(std::max(fewest, std::min(most, positions * groups * n_layers / kSharedItems))));
+  return HEXKV_OK;
+}
+
+extern "C" int hexkv_attend_layers_independent(const hexkv_attend_params *p, const hexkv_attend_layer *layers,
+                                               int n_layers) {
+  using namespace hexkv;
+  clear_error();
+  if (!p || n_layers < 1 || !layers || p->batch < 1) return 0;
+  return layers_independent(p, layers, n_layers) ? 1 : 0;
+}
+
+namespace hexkv {
+
 // The work list of a planning request, in launch order (see hexkv_attend_plan),
 // and each (row, head group) segment's partition count.
 static int build_plan(const hexkv_attend_params *p, const int32_t *lens, int64_t chunk,
@@ -2106,16 +2212,89 @@ static int run_tiles(const hexkv_attend_params *p, const AttendArgs &a, hipStrea
   return check_launch(what);
 }
 
-// The launch behind hexkv_attend and hexkv_attend_noalloc: validated
-// parameters, a workspace of ws_bytes bytes (device memory), one stream.
-static int attend_launch(const hexkv_attend_params *p, void *workspace, size_t ws_bytes,
-                         hexkv_stream_t stream, const char *what) {
+// Slots (partials of D outputs and a (max, sum) pair) of one call.
+static int64_t workspace_slots(const hexkv_attend_params *p, int64_t max_parts) {
+  return static_cast<int64_t>(p->batch) * p->q_len * p->q_heads * max_parts;
+}
+
+// Whether split segments of this call merge in the attention kernel: a list
+// planned for the XCDs whose segments one workgroup can merge (the row-block
+// kernel's always: validate() holds it to such lists).
+static bool merges_in_kernel(const hexkv_attend_params *p, int64_t max_parts) {
+  return p->work_items_dev && p->work_xcds > 0 && p->work_xcds <= 8 && max_parts <= kMergeMaxParts &&
+         (p->kernel == HEXKV_KERNEL_ROWS ||
+          kernel_group(p->q_heads / p->kv_heads) * p->head_dim <= 4 * kAttThreads);
+}
+
+// Layers of one geometry that one launch may hold (1: one launch each): a
+// list dealt over whole rounds of XCDs, so a segment's items stay on one XCD
+// in every layer, whose split segments merge in the kernel and whose arrival
+// counters fit, short enough that the layer does not fill the chip several
+// times over by itself (see kSharedLayerBytes).
+constexpr int32_t kSharedListItems = 1024;
+
+static int64_t layers_per_launch(const hexkv_attend_params *p, int n_layers) {
+  const int64_t max_parts = max_parts_of(p, 1);
+  if (!p->work_items_dev || p->work_xcds < 1 || p->n_work_items % p->work_xcds ||
+      p->n_work_items > kSharedListItems ||
+      (max_parts > 1 && !merges_in_kernel(p, max_parts)))
+    return 1;
+  const int64_t segs = static_cast<int64_t>(p->batch) * (p->q_heads / segment_heads(p));
+  const int64_t fit = max_parts > 1 ? kCounterWords / std::max<int64_t>(1, segs) : n_layers;
+  return std::max<int64_t>(1, std::min<int64_t>({fit, n_layers, 65535}));
+}
+
+// Whether no layer writes bytes that another layer reads or writes (each
+// tensor counted as its whole extent), so their order does not matter.
+static bool layers_independent(const hexkv_attend_params *p, const hexkv_attend_layer *layers, int n_layers) {
+  struct Extent {
+    uintptr_t lo, hi;
+    int layer;
+    bool write;
+  };
+  const int64_t es = elem_size(p->dtype), row = static_cast<int64_t>(p->q_heads) * p->head_dim;
+  const int64_t kv_row = static_cast<int64_t>(p->kv_heads) * p->head_dim;
+  const auto span = [&](int64_t batch_stride, int64_t inner) {
+    return static_cast<uintptr_t>(((p->batch - 1) * batch_stride + inner) * es);
+  };
+  std::vector<Extent> e;
+  e.reserve(4 * static_cast<size_t>(n_layers) + 1);
+  const auto add = [&](const void *base, uintptr_t bytes, int layer, bool write) {
+    const uintptr_t lo = reinterpret_cast<uintptr_t>(base);
+    if (base) e.push_back(Extent{lo, lo + bytes, layer, write});
+  };
+  if (p->capacity < 1 || p->q_batch_stride < 0 || p->out_batch_stride < 0 || p->cache_batch_stride < 0) return false;
+  for (int l = 0; l < n_layers; ++l) {
+    add(layers[l].q, span(p->q_batch_stride, row), l, false);
+    add(layers[l].kv_new, span(2 * kv_row, 2 * kv_row), l, false);
+    add(layers[l].out, span(p->out_batch_stride, row), l, true);
+    add(layers[l].cache, span(p->cache_batch_stride, (p->capacity - 1) * p->cache_pos_stride + p->cache_kv_stride + kv_row),
+        l, true);
+  }
+  add(p->lengths_out_dev, p->batch * sizeof(int32_t), n_layers - 1, true);
+  std::sort(e.begin(), e.end(), [](const Extent &a, const Extent &b) { return a.lo < b.lo; });
+  // Two layers' extents that overlap, one of them written: seen when the
+  // later one starts below the furthest end of another layer's.
+  for (size_t i = 0; i < e.size(); ++i)
+    for (size_t j = i + 1; j < e.size() && e[j].lo < e[i].hi; ++j)
+      if (e[i].layer != e[j].layer && (e[i].write || e[j].write)) return false;
+  return true;
+}
+
+// The launch behind hexkv_attend, hexkv_attend_noalloc and
+// hexkv_attend_layers: validated parameters, a workspace of ws_bytes bytes
+// (device memory), one stream.  `layers` (device memory): n_layers
+// independent layers in one launch (layers_per_launch allows them), else
+// nullptr and the layer in `p`.
+static int attend_launch(const hexkv_attend_params *p, void *workspace, size_t ws_bytes, hexkv_stream_t stream,
+                         const char *what, const hexkv_attend_layer *layers = nullptr, int n_layers = 1) {
   int rc = validate(p);
   if (rc != HEXKV_OK || p->batch == 0) return rc;
   const int part = partition_of(p);
   const int G = kernel_group(p->q_heads / p->kv_heads);
   const int64_t max_parts = max_parts_of(p, part);
-  const size_t need = workspace_bytes(p, part);
+  const size_t one = workspace_bytes(p, part);
+  const size_t need = one ? one + (n_layers - 1) * (one - HEXKV_ATTEND_COUNTER_BYTES) : 0;
   if (need > 0 && (!workspace || ws_bytes < need))
     return fail(HEXKV_EWORKSPACE, "%s: workspace of %zu bytes needed, %zu given", what, need, ws_bytes);
   if (need > 0 && !aligned16(workspace))
@@ -2150,19 +2329,17 @@ static int attend_launch(const hexkv_attend_params *p, void *workspace, size_t w
   a.ws_ml = nullptr;
   if (need > 0) {
     a.ws_o = reinterpret_cast<float *>(static_cast<char *>(workspace) + HEXKV_ATTEND_COUNTER_BYTES);
-    a.ws_ml = a.ws_o + rows * p->q_heads * max_parts * p->head_dim;
+    a.ws_ml = a.ws_o + n_layers * workspace_slots(p, max_parts) * p->head_dim;
   }
+  a.layers = layers;
+  a.layer_slots = need > 0 ? workspace_slots(p, max_parts) : 0;
   const bool rows_kernel = p->kernel == HEXKV_KERNEL_ROWS;
   a.n_groups = p->q_heads / segment_heads(p);
   a.rows = static_cast<int32_t>(rows);
   a.items = p->work_items_dev;
   a.seg_parts = p->work_parts_dev;
-  // Split segments of a list planned for the XCDs merge in the attention
-  // kernel, counting arrivals in the workspace's counter words (the
-  // row-block kernel's always: validate() holds it to such lists).
-  a.seg_count = (a.items && p->work_xcds > 0 && p->work_xcds <= 8 && need > 0 && max_parts <= kMergeMaxParts &&
-                 (rows_kernel || G * p->head_dim <= 4 * kAttThreads))
-                    ? static_cast<uint64_t *>(workspace) : nullptr;
+  // Arrivals at a merge in the kernel count in the workspace's counter words.
+  a.seg_count = need > 0 && merges_in_kernel(p, max_parts) ? static_cast<uint64_t *>(workspace) : nullptr;
   a.n_xcd = p->work_xcds;
   a.xcd_remap = 0;
   if (a.items && p->work_xcds > 0) {
@@ -2186,7 +2363,8 @@ static int attend_launch(const hexkv_attend_params *p, void *workspace, size_t w
 
   dim3 grid;
   if (a.items) {
-    grid = dim3(static_cast<unsigned>(p->n_work_items));  // one workgroup per item, in list order
+    // one workgroup per item, in list order, layer by layer
+    grid = dim3(static_cast<unsigned>(p->n_work_items), static_cast<unsigned>(n_layers));
   } else {
     // Workgroups reach the 8 XCDs round-robin by linear index, and the later
     // partitions exist only in long rows.  With an even partition count the
@@ -2235,6 +2413,65 @@ extern "C" int hexkv_attend(const hexkv_attend_params *p, void *workspace, size_
                             hexkv_stream_t stream) {
   hexkv::clear_error();
   return hexkv::attend_launch(p, workspace, ws_bytes, stream, "hexkv_attend");
+}
+
+// Workspace of a multi-layer launch above which the layers go in several.
+static constexpr size_t kLayersWorkspace = size_t{256} << 20;
+
+extern "C" size_t hexkv_attend_layers_workspace_bytes(const hexkv_attend_params *p, const hexkv_attend_layer *layers,
+                                                      int n_layers) {
+  using namespace hexkv;
+  const size_t one = hexkv_attend_workspace_bytes(p);
+  if (one == 0 || !layers || n_layers < 2 || p->batch < 1) return one;
+  const int64_t most = layers_per_launch(p, n_layers);
+  if (most < 2 || !layers_independent(p, layers, n_layers)) return one;
+  const size_t per = one - HEXKV_ATTEND_COUNTER_BYTES;
+  const size_t fit = std::max<size_t>(1, (kLayersWorkspace - HEXKV_ATTEND_COUNTER_BYTES) / per);
+  return HEXKV_ATTEND_COUNTER_BYTES + std::min<size_t>(fit, static_cast<size_t>(most)) * per;
+}
+
+extern "C" int hexkv_attend_layers(const hexkv_attend_params *p, const hexkv_attend_layer *layers,
+                                   const hexkv_attend_layer *layers_dev, int n_layers, void *workspace,
+                                   size_t ws_bytes, hexkv_stream_t stream) {
+  using namespace hexkv;
+  clear_error();
+  const char *what = "hexkv_attend_layers";
+  if (!p || n_layers < 0 || (n_layers > 0 && !layers)) return fail(HEXKV_EINVAL, "%s: null argument", what);
+  const auto layer = [&](int l) {
+    hexkv_attend_params q = *p;
+    q.q = layers[l].q;
+    q.cache = layers[l].cache;
+    q.out = layers[l].out;
+    q.kv_new = layers[l].kv_new;
+    if (l + 1 < n_layers) q.lengths_out_dev = nullptr;
+    return q;
+  };
+  for (int l = 0; l < n_layers; ++l) {
+    if ((layers[l].kv_new == nullptr) != (layers[0].kv_new == nullptr))
+      return fail(HEXKV_EINVAL, "%s: kv_new in some layers only", what);
+    const hexkv_attend_params q = layer(l);
+    const int rc = validate(&q);
+    if (rc != HEXKV_OK) return rc;
+  }
+  if (n_layers == 0 || p->batch == 0) return HEXKV_OK;
+  // As many layers a launch as the counters and this workspace hold.
+  int64_t per_launch = 1;
+  if (n_layers > 1 && layers_dev && aligned16(layers_dev) && layers_independent(p, layers, n_layers)) {
+    per_launch = layers_per_launch(p, n_layers);
+    const size_t one = workspace_bytes(p, 1);
+    if (one > 0) {
+      const size_t per = one - HEXKV_ATTEND_COUNTER_BYTES;
+      const size_t fit = ws_bytes > HEXKV_ATTEND_COUNTER_BYTES ? (ws_bytes - HEXKV_ATTEND_COUNTER_BYTES) / per : 0;
+      per_launch = std::max<int64_t>(1, std::min<int64_t>(per_launch, static_cast<int64_t>(fit)));
+    }
+  }
+  for (int l = 0; l < n_layers; l += static_cast<int>(per_launch)) {
+    const int n = static_cast<int>(std::min<int64_t>(per_launch, n_layers - l));
+    const hexkv_attend_params q = layer(l + n - 1);  // the last of a launch records the lengths
+    const int rc = attend_launch(&q, workspace, ws_bytes, stream, what, n > 1 ? layers_dev + l : nullptr, n);
+    if (rc != HEXKV_OK) return rc;
+  }
+  return HEXKV_OK;
 }
 
 extern "C" int hexkv_attend_noalloc(const hexkv_attend_params *p, hexkv_stream_t stream) {

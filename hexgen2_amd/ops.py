@@ -792,9 +792,14 @@ class AttendPlan:
         self.lens = None if lens is None else [int(n) for n in lens]
         self.work_key, self.work = None, None
         self.kernel = self.params.kernel  # as requested; a work list sets the one its launches use
+        self.layers = None  # set_layers: (tensors, host table, device table)
 
     def _grow_workspace(self) -> None:
-        need = int(self.lib.hexkv_attend_workspace_bytes(ctypes.byref(self.params)))
+        if self.layers is None:
+            need = int(self.lib.hexkv_attend_workspace_bytes(ctypes.byref(self.params)))
+        else:
+            table = self.layers[1]
+            need = int(self.lib.hexkv_attend_layers_workspace_bytes(ctypes.byref(self.params), table, len(table)))
         if need > self.ws_bytes:
             self.workspace = torch.zeros(need, dtype=torch.uint8, device=self.device)
             self.ws_ptr, self.ws_bytes = self.workspace.data_ptr(), need
@@ -861,6 +866,40 @@ class AttendPlan:
         return out
 
 
+    def set_layers(self, q: Sequence[torch.Tensor], cache: Sequence[torch.Tensor], out: Sequence[torch.Tensor],
+                   kv_new: Sequence[torch.Tensor]) -> None:
+        """Fix the layers ``call_layers`` runs (each of the plan's geometry;
+        kept alive with the plan) and write their addresses to device memory."""
+        for tensors in zip(q, cache, out, kv_new):
+            self.check(*tensors)
+        table = (_lib.AttendLayer * len(q))(*[tuple(t.data_ptr() for t in tensors)
+                                              for tensors in zip(q, cache, out, kv_new)])
+        device_table = torch.frombuffer(table, dtype=torch.int64).clone().to(self.device)
+        self.layers = (list(q), list(cache), list(out), list(kv_new)), table, device_table
+
+    def shared_layers(self) -> int:
+        """How many of the set layers may share a launch: all of them when no
+        layer writes what another reads or writes, else 1."""
+        _, table, _ = self.layers
+        return len(table) if self.lib.hexkv_attend_layers_independent(ctypes.byref(self.params), table,
+                                                                      len(table)) else 1
+
+    def call_layers(self, seqlen_bias: int, max_seqlen: int, lengths_out: torch.Tensor) -> None:
+        """One call per layer of ``set_layers`` in order, over the fixed work
+        list, the last with ``lengths_out``; layers whose tensors do not
+        overlap share launches (``hexkv_attend_layers``)."""
+        p = self.params
+        _, table, device_table = self.layers
+        p.seqlen_bias, p.max_seqlen = int(seqlen_bias), int(max_seqlen)
+        p.lengths_out_dev = lengths_out.data_ptr()
+        try:
+            rc = self.lib.hexkv_attend_layers(ctypes.byref(p), table, device_table.data_ptr(), len(table),
+                                              self.ws_ptr, self.ws_bytes, _stream(device_table))
+        finally:
+            p.lengths_out_dev = None
+        _lib.check(rc, "hexkv_attend_layers")
+
+
 class StepWorkLists:
     """The work lists of consecutive decode steps, planned once on the host
     and kept in one device buffer.
@@ -871,12 +910,13 @@ class StepWorkLists:
     one) and, with ``single_launch``, for the device's XCDs.  ``self[t]`` is
     step t's ``WorkList``; ``chunks[t]`` its chunk and ``kernels[t]`` the
     kernel value it was planned with (``hexkv_attend_plan_kernel``: the
-    row-block kernel for "auto" on large calls).  Nothing is planned or
-    copied per step afterwards.
+    row-block kernel for "auto" on large calls).  ``layers``: how many layers
+    share each list's launches (``hexkv_attend_plan_layers``).  Nothing is
+    planned or copied per step afterwards.
     """
 
     def __init__(self, p: _lib.AttendParams, lens: Sequence[int], steps: int, device,
-                 single_launch: bool = True, partition: int = 0):
+                 single_launch: bool = True, partition: int = 0, layers: int = 1):
         if torch.cuda.is_current_stream_capturing():
             raise ValueError("StepWorkLists must be built before graph capture")
         lib = _lib.load()
@@ -895,12 +935,15 @@ class StepWorkLists:
         requested = q.kernel
         sizes, self.chunks, self.kernels = [], [], []
         for t in range(steps):
-            q.seqlen_bias, q.kernel, q.partition = t, requested, 0
-            q.kernel = _plan_kernel(q, c_lens)
-            chunk, n, mp = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
-            q.partition = int(partition)
-            _lib.check(lib.hexkv_attend_plan_chunk(ctypes.byref(q), c_lens, ctypes.byref(chunk)),
-                       "hexkv_attend_plan_chunk")
+            q.seqlen_bias, q.kernel, q.partition = t, requested, int(partition)
+            kern, chunk, n, mp = ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32(), ctypes.c_int32()
+            if q.partition and q.kernel == _lib.KERNELS["auto"]:
+                q.partition = 0  # the kernel is chosen before the chunk's grain is known
+                q.kernel = _plan_kernel(q, c_lens)
+                q.partition = int(partition)
+            _lib.check(lib.hexkv_attend_plan_layers(ctypes.byref(q), c_lens, max(int(layers), 1), ctypes.byref(kern),
+                                                    ctypes.byref(chunk)), "hexkv_attend_plan_layers")
+            q.kernel = kern.value
             q.partition = chunk.value
             _lib.check(lib.hexkv_attend_plan(ctypes.byref(q), c_lens, None, 0, None, 0, ctypes.byref(n),
                                              ctypes.byref(mp)), "hexkv_attend_plan")
@@ -983,8 +1026,7 @@ class DecodeStepGraph:
                                seqlens=positions, kv_new=self.kv_new[0], softmax_scale=softmax_scale,
                                kernel=kernel, partition=partition)
         # Every layer is checked before anything is captured.
-        for l in range(len(self.q)):
-            self.plan.check(self.q[l], self.cache[l], self.out[l], self.kv_new[l])
+        self.plan.set_layers(self.q, self.cache, self.out, self.kv_new)
         self.lists = None
         self.step = 0
         if lens is None:
@@ -997,18 +1039,18 @@ class DecodeStepGraph:
         steps = self.max_seqlen - max([int(n) for n in lens], default=0)
         if steps < 1:
             raise ValueError(f"max_seqlen {max_seqlen} leaves no step for lengths up to {max(lens)}")
-        self.lists = StepWorkLists(self.plan.params, lens, steps, positions.device, single_launch, partition)
+        self.lists = StepWorkLists(self.plan.params, lens, steps, positions.device, single_launch, partition,
+                                   self.plan.shared_layers())
         self.plan.reserve(self.lists.lists)
         self.graphs = []
         pool = None
-        last = len(self.q) - 1
+        if positions.numel() < self.plan.params.batch:
+            raise ValueError("positions must have one entry per sequence")
         for t in range(steps):
             self.plan.fix_work_list(self.lists[t])
             graph = torch.cuda.CUDAGraph()
             with torch.cuda.graph(graph, pool=pool):
-                for l in range(len(self.q)):
-                    self.plan(self.q[l], self.cache[l], self.out[l], self.kv_new[l], 0, self.max_seqlen,
-                              lengths_out=self.positions if l == last else None)
+                self.plan.call_layers(0, self.max_seqlen, lengths_out=self.positions)
             pool = graph.pool()
             self.graphs.append(graph)
 

@@ -294,6 +294,37 @@ int hexkv_attend_kernel(const hexkv_attend_params *p);
 int hexkv_attend(const hexkv_attend_params *p, void *workspace,
                  size_t workspace_bytes, hexkv_stream_t stream);
 
+/* The tensors of one layer of a hexkv_attend_layers call (device memory). */
+typedef struct hexkv_attend_layer {
+  const void *q;
+  void *cache;
+  void *out;
+  const void *kv_new;
+} hexkv_attend_layer;
+
+/*
+ * hexkv_attend for n_layers layers that share p's geometry, lengths and work
+ * list (p's own q, cache, out and kv_new are not read), with the results of
+ * n_layers calls in order; p->lengths_out_dev is written by the last layer.
+ * `layers` is host memory; `layers_dev`, a 16-byte aligned copy of it in
+ * device memory that must outlive the work, lets layers whose tensors do not
+ * overlap share launches: work lists planned for the XCDs (work_xcds > 0),
+ * as many layers a launch as the arrival counters and the workspace hold.
+ * Any other call, or layers_dev NULL, or a list of more than 1024 items, is
+ * n_layers launches.
+ * hexkv_attend_layers_workspace_bytes returns the workspace that lets the
+ * most layers share (never above 256 MiB for several); hexkv_attend's for
+ * one layer is the least.  No counterpart in the reference.
+ */
+/* 1 if no layer writes bytes another one reads or writes (each tensor taken
+ * as its whole extent), else 0. */
+int hexkv_attend_layers_independent(const hexkv_attend_params *p, const hexkv_attend_layer *layers, int n_layers);
+size_t hexkv_attend_layers_workspace_bytes(const hexkv_attend_params *p, const hexkv_attend_layer *layers,
+                                           int n_layers);
+int hexkv_attend_layers(const hexkv_attend_params *p, const hexkv_attend_layer *layers,
+                        const hexkv_attend_layer *layers_dev, int n_layers, void *workspace,
+                        size_t workspace_bytes, hexkv_stream_t stream);
+
 /*
  * Work list for hexkv_attend over decode rows whose lengths the host knows:
  * row b attends len_b = lens[b] + p->seqlen_bias (+1 with kv_new) keys,
@@ -360,6 +391,13 @@ int hexkv_attend_plan_chunk(const hexkv_attend_params *p, const int32_t *lens, i
  * step).
  */
 int hexkv_attend_plan_kernel(const hexkv_attend_params *p, const int32_t *lens, int32_t *kernel);
+
+/* Kernel and chunk to plan a list with that n_layers layers of a
+ * hexkv_attend_layers call share: hexkv_attend_plan_kernel's and
+ * hexkv_attend_plan_chunk's for one layer.  An explicit p->kernel or
+ * p->partition is kept. */
+int hexkv_attend_plan_layers(const hexkv_attend_params *p, const int32_t *lens, int n_layers, int32_t *kernel,
+                             int32_t *chunk);
 
 /* Size of the static scratch array behind hexkv_attend_noalloc (per GPU). */
 #define HEXKV_NOALLOC_SCRATCH_BYTES (32u << 20)

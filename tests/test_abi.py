@@ -40,7 +40,8 @@ def test_library_exports_every_declared_symbol():
                                             ("hexkv_ft_attend_params", _lib.FtAttendParams),
                                             ("hexkv_block", _lib.Block),
                                             ("hexkv_ipc_handle", _lib.IpcHandle),
-                                            ("hexkv_work_item", _lib.WorkItem)])
+                                            ("hexkv_work_item", _lib.WorkItem),
+                                            ("hexkv_attend_layer", _lib.AttendLayer)])
 def test_struct_layouts_match_c(tmp_path, c_name, mirror):
     fields = [f[0] for f in mirror._fields_]
     src = tmp_path / "layout.c"

@@ -1,0 +1,72 @@
+"""Planning of lists that several layers share, on the host: one layer gets
+the one-layer rules, several a chunk that every kernel accepts; and the check
+for layers whose tensors overlap."""
+import ctypes
+
+import pytest
+
+from hexgen2_amd import _lib
+
+
+def _params(dtype, batch, hq, hkv, d, longest, kernel=0, xcds=8):
+    return _lib.AttendParams(dtype=dtype, batch=batch, q_len=1, q_heads=hq, kv_heads=hkv, head_dim=d, softmax_scale=1.0,
+                             capacity=longest + 1, max_seqlen=longest + 1, kv_new=16, kernel=kernel, work_xcds=xcds)
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d", [(0, 32, 4, 64), (0, 32, 32, 128), (1, 8, 1, 128), (1, 32, 8, 128), (2, 4, 4, 16)])
+@pytest.mark.parametrize("lens", [[0], [1], [5000], [64, 8192, 17], [2048] * 8, [8192] * 64])
+@pytest.mark.parametrize("layers", [1, 2, 16, 80])
+def test_plan_layers(dtype, hq, hkv, d, lens, layers):
+    lib = _lib.load()
+    p = _params(dtype, len(lens), hq, hkv, d, max(lens))
+    c = (ctypes.c_int32 * len(lens))(*lens)
+    kernel, chunk, one_kernel, one_chunk = (ctypes.c_int32() for _ in range(4))
+    assert lib.hexkv_attend_plan_layers(p, c, layers, kernel, chunk) == 0
+    assert lib.hexkv_attend_plan_kernel(p, c, one_kernel) == 0
+    p.kernel = one_kernel.value
+    assert lib.hexkv_attend_plan_chunk(p, c, one_chunk) == 0
+    if layers == 1 or len(lens) == 64 and hkv >= 8 and d == 128:  # a layer of 512 MB or more runs alone
+        assert (kernel.value, chunk.value) == (one_kernel.value, one_chunk.value)
+    # the list can be built with it, and its segments merge in the kernel
+    p.kernel, p.partition = kernel.value, chunk.value
+    n, most = ctypes.c_int32(), ctypes.c_int32()
+    assert lib.hexkv_attend_plan(p, c, None, 0, None, 0, n, most) == 0
+    assert n.value % 8 == 0 and (layers == 1 or most.value <= 64)
+
+
+def test_plan_layers_keeps_what_the_caller_chose():
+    lib = _lib.load()
+    p = _params(0, 2, 32, 32, 128, 4000, kernel=1)
+    p.partition = 192
+    c = (ctypes.c_int32 * 2)(4000, 3000)
+    kernel, chunk = ctypes.c_int32(), ctypes.c_int32()
+    assert lib.hexkv_attend_plan_layers(p, c, 8, kernel, chunk) == 0
+    assert (kernel.value, chunk.value) == (1, 192)
+    assert lib.hexkv_attend_plan_layers(p, c, 0, kernel, chunk) == _lib.HEXKV_EINVAL
+
+
+@pytest.mark.parametrize("change,free", [(None, 1), ("out", 0), ("cache", 0), ("q", 1), ("q_in_out", 0), ("kv_in_cache", 0),
+                                         ("touching", 1), ("lengths", 0)])
+def test_layers_independent(change, free):
+    """Only written bytes shared between layers force an order."""
+    lib = _lib.load()
+    batch, cap, hkv, hq, d = 2, 64, 2, 4, 64
+    p = _params(0, batch, hq, hkv, d, cap - 1)
+    p.q_batch_stride = p.out_batch_stride = hq * d
+    p.cache_batch_stride, p.cache_pos_stride, p.cache_kv_stride = cap * 2 * hkv * d, 2 * hkv * d, hkv * d
+    p.capacity = cap
+    cache, row, new = batch * cap * 2 * hkv * d * 2, batch * hq * d * 2, batch * 2 * hkv * d * 2
+    base = 1 << 20
+    a = _lib.AttendLayer(base, base + (1 << 20), base + (2 << 20), base + (3 << 20))
+    b = _lib.AttendLayer(base + (4 << 20), base + (5 << 20), base + (6 << 20), base + (7 << 20))
+    if change in ("out", "cache", "q"):
+        setattr(b, change, getattr(a, change))
+    elif change == "q_in_out":
+        b.q = a.out + row - 16
+    elif change == "kv_in_cache":
+        b.kv_new = a.cache + cache - new
+    elif change == "touching":
+        b.q, b.kv_new, b.out, b.cache = a.out + row, a.cache + cache, a.out - row, a.cache - cache
+    elif change == "lengths":
+        p.lengths_out_dev = a.out + 8
+    assert lib.hexkv_attend_layers_independent(p, (_lib.AttendLayer * 2)(a, b), 2) == free
