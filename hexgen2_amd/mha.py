@@ -63,10 +63,15 @@ def _sample_positions(inference_params, batch_start: int, batch_end: int) -> Opt
     if lengths.dim() != 1 or lengths.shape[0] < batch_end:
         raise ValueError(f"lengths_per_sample of shape {tuple(lengths.shape)} does not cover "
                          f"sequences [{batch_start}, {batch_end})")
-    positions = lengths[batch_start:batch_end]
+    positions = _batch_rows(lengths, batch_start, batch_end)
     if positions.dtype != torch.int32 or not positions.is_contiguous():
         positions = positions.to(torch.int32).contiguous()
     return positions
+
+
+def _batch_rows(cache: torch.Tensor, start: int, end: int) -> torch.Tensor:
+    """``cache[start:end]``, without building a view of the whole cache."""
+    return cache if start == 0 and end == cache.shape[0] else cache[start:end]
 
 
 def _update_kv_cache(kv: torch.Tensor, inference_params, layer_idx: int) -> torch.Tensor:
@@ -103,16 +108,13 @@ def _update_kv_cache(kv: torch.Tensor, inference_params, layer_idx: int) -> torc
     assert batch_end <= cache.shape[0]
     assert sequence_end <= cache.shape[1]
     kv = kv.contiguous()
-    target = cache[batch_start:batch_end]
     positions = _sample_positions(inference_params, batch_start, batch_end) if kv.shape[1] == 1 else None
     if positions is not None:
-        ops.append_kv(target, kv.reshape(kv.shape[0], -1), positions)
+        ops.append_kv(_batch_rows(cache, batch_start, batch_end), kv, positions)
     elif kv.shape[1] == 1:
-        ops.append_kv(target, kv.reshape(kv.shape[0], -1), position_bias=sequence_start)
+        ops.append_kv(_batch_rows(cache, batch_start, batch_end), kv, position_bias=sequence_start)
     elif kv.shape[1] > 1:
-        # A multi-position write (prefill) is an unpack of one packed layer with
-        # uniform lengths into the cache shifted by sequence_start rows.
-        ops.unpack_live([kv.reshape(-1)], [target[:, sequence_start:]], [kv.shape[1]] * kv.shape[0])
+        ops.write_rows(cache, kv, batch_start, sequence_start)
     view = cache[batch_start:batch_end, :sequence_end]
     if positions is not None:
         setattr(view, _SEQLENS_ATTR, (positions, 1))
@@ -223,7 +225,7 @@ class FlashCrossAttention(nn.Module):
             assert seqlens_k.dtype == torch.int32 and seqlens_k.is_cuda and seqlens_k.numel() == batch_size
             seqlens_k = seqlens_k.contiguous()
         q = q if q.stride(-1) == 1 and q.stride(-2) == q.shape[-1] else q.contiguous()
-        if kv.stride(-1) != 1 or kv.stride(-2) != kv.shape[-1] or kv.stride(1) != kv[0, 0].numel():
+        if kv.stride(-1) != 1 or kv.stride(-2) != kv.shape[-1] or kv.stride(1) != kv.shape[2:].numel():
             kv = kv.contiguous()
         return ops.decode_attention(q, kv, max_seqlen=seqlen_k, seqlens=seqlens_k, seqlen_bias=bias,
                                     causal=bool(causal) and q.shape[1] > 1,
@@ -254,7 +256,7 @@ def update_and_attend(q: torch.Tensor, kv: torch.Tensor, inference_params, layer
     offset = inference_params.sequence_len_offset
     assert kv.shape[1] == 1 and q.shape[1] == 1
     assert batch_end <= cache.shape[0] and offset + 1 <= cache.shape[1]
-    target = cache[batch_start:batch_end]
+    target = _batch_rows(cache, batch_start, batch_end)
     positions = _sample_positions(inference_params, batch_start, batch_end)
     return ops.decode_attention(q.contiguous(), target, max_seqlen=offset + 1, seqlens=positions,
                                 seqlen_bias=0 if positions is not None else offset,

@@ -265,6 +265,29 @@ def unpack_live(packed: TensorList, cache_layers: TensorList, lens: Sequence[int
     _lib.check(rc, "hexkv_unpack")
 
 
+def write_rows(cache: torch.Tensor, kv: torch.Tensor, batch_start: int, start: int) -> None:
+    """Write the positions of ``kv [b, s, *row]`` (contiguous) at
+    ``cache[batch_start:batch_start + b, start:start + s]`` (``[B, S, *row]``):
+    the multi-position write of hexgen/hexgen_core/modules/mha.py:286, one
+    launch of the unpack kernel over one layer with uniform lengths."""
+    _require_device(cache, kv)
+    batch, seqlen = kv.shape[:2]
+    stride, elem = cache.stride(), cache.element_size()
+    # the geometry of the written sequences alone: one needs no whole-row batch stride
+    row_elems, row_bytes, seq_stride = _row_geometry_of((batch, *cache.shape[1:]), stride, elem)
+    if kv.dtype != cache.dtype or kv.device != cache.device:
+        raise ValueError("kv and cache differ in dtype or device")
+    if kv.numel() != batch * seqlen * row_elems or not kv.is_contiguous():
+        raise ValueError(f"kv must be contiguous [batch, positions, *row], got {tuple(kv.shape)}")
+    if batch_start < 0 or batch_start + batch > cache.shape[0] or start < 0 or start + seqlen > cache.shape[1]:
+        raise ValueError("rows outside the cache")
+    base = cache.data_ptr() + batch_start * stride[0] * elem + start * row_bytes
+    rc = _lib.load().hexkv_unpack((ctypes.c_void_p * 1)(kv.data_ptr()), (ctypes.c_void_p * 1)(base), 1, batch,
+                                  seq_stride, cache.shape[1] - start, row_bytes,
+                                  (ctypes.c_int64 * batch)(*([seqlen] * batch)), _stream(cache))
+    _lib.check(rc, "hexkv_unpack")
+
+
 def append_kv(cache: torch.Tensor, kv_new: torch.Tensor, positions: Optional[torch.Tensor] = None,
               position_bias: int = 0) -> None:
     """Write ``kv_new[b]`` (one row per sequence) into ``cache[b, pos_b]`` with
@@ -386,25 +409,70 @@ def decode_attention(q: torch.Tensor, cache: torch.Tensor, *, max_seqlen: int,
     after allocation (its leading counter words; every call leaves them zero).
     """
     _require_device(q, cache)
-    if out is None:
-        out = torch.empty(q.shape, dtype=q.dtype, device=q.device)
-    p = _attend_params(q, cache, out, seqlens, seqlen_bias, max_seqlen, kv_new, causal,
-                       softmax_scale, partition, kernel)
     lib = _lib.load()
+    softmax_scale = None if softmax_scale is None else float(softmax_scale)
+    key = (_tensor_geometry(q), _tensor_geometry(cache), _tensor_geometry(out), _tensor_geometry(kv_new),
+           _tensor_geometry(seqlens), bool(causal), softmax_scale, int(partition), kernel)
+    if out is None:
+        out = q.new_empty(q.shape)
+    form = _ATTEND_FORMS.get(key)
+    if form is None:
+        p = _attend_params(q, cache, out, seqlens, seqlen_bias, max_seqlen, kv_new, causal,
+                           softmax_scale, partition, kernel)
+        _keep_form(key, p)
+        needs = None
+    else:
+        p = _lib.AttendParams.from_buffer_copy(form[0])
+        needs = form[1]
+        p.q, p.cache, p.out = q.data_ptr(), cache.data_ptr(), out.data_ptr()
+        if kv_new is not None:
+            p.kv_new = kv_new.data_ptr()
+        if seqlens is not None:
+            p.seqlens_dev = seqlens.data_ptr()
+        p.seqlen_bias, p.max_seqlen = int(seqlen_bias), int(max_seqlen)
     work = None
     if lens is not None:
         work = _plan_work(p, lens, q.device, single_launch)  # kept alive until the launch is enqueued
         work.apply(p)
-    need = int(lib.hexkv_attend_workspace_bytes(ctypes.byref(p)))
+    if work is not None or needs is None:
+        need = int(lib.hexkv_attend_workspace_bytes(ctypes.byref(p)))
+    else:
+        need = needs.get(p.max_seqlen)
+        if need is None:
+            need = int(lib.hexkv_attend_workspace_bytes(ctypes.byref(p)))
+            if len(needs) >= 64:
+                needs.clear()
+            needs[p.max_seqlen] = need
     ws_ptr, ws_bytes = None, 0
     if need:
         if workspace is None or workspace.numel() * workspace.element_size() < need:
-            workspace = torch.zeros(need, dtype=torch.uint8, device=q.device)
+            # only a work list's merge counts in the workspace and needs it zero
+            make = torch.empty if work is None else torch.zeros
+            workspace = make(need, dtype=torch.uint8, device=q.device)
         _require_device(workspace)
         ws_ptr, ws_bytes = workspace.data_ptr(), workspace.numel() * workspace.element_size()
     rc = lib.hexkv_attend(ctypes.byref(p), ws_ptr, ws_bytes, _stream(q))
     _lib.check(rc, "hexkv_attend")
     return out
+
+
+# decode_attention's checked parameter blocks by what they depend on: every
+# tensor's shape, strides, dtype and device, and the options, never an
+# address.  (block, {max_seqlen: workspace bytes}) each; the addresses and
+# lengths of a call go into a copy.  Building and checking the block anew
+# was about 9 of an eager decode layer's 20 us of host time.
+_ATTEND_FORMS: "OrderedDict[tuple, tuple]" = OrderedDict()
+
+
+def _keep_form(key: tuple, p: _lib.AttendParams) -> None:
+    form = _lib.AttendParams.from_buffer_copy(p)
+    form.q = form.cache = form.out = form.kv_new = form.seqlens_dev = None
+    _ATTEND_FORMS[key] = form, {}
+    while len(_ATTEND_FORMS) > 64:
+        try:
+            _ATTEND_FORMS.popitem(last=False)
+        except KeyError:  # another thread emptied it
+            break
 
 
 class WorkList:
