@@ -50,6 +50,17 @@ __device__ __forceinline__ Pack<T, VEC> norm_input(const NormArgs &a, int64_t ro
   return v;
 }
 
+template <typename T, int VEC>
+__device__ __forceinline__ Pack<T, VEC> norm_scale(const Pack<T, VEC> &v, const Pack<T, VEC> &w, float r) {
+  Pack<T, VEC> o;
+#pragma unroll
+  for (int k = 0; k < VEC; ++k) {
+    const T n = Elem<T>::from_float(static_cast<float>(v.e[k]) * r);
+    o.e[k] = Elem<T>::from_float(static_cast<float>(n) * static_cast<float>(w.e[k]));
+  }
+  return o;
+}
+
 template <typename T, int VEC, int NV>
 __global__ __launch_bounds__(kLayerThreads) void add_rms_norm_kernel(const NormArgs a) {
   using P = Pack<T, VEC>;
@@ -85,13 +96,7 @@ __global__ __launch_bounds__(kLayerThreads) void add_rms_norm_kernel(const NormA
   T *out = static_cast<T *>(a.out) + row * a.hidden;
   auto scale = [&](const P &v, int i) {
     const P w = *reinterpret_cast<const P *>(static_cast<const T *>(a.weight) + i);
-    P o;
-#pragma unroll
-    for (int k = 0; k < VEC; ++k) {
-      const T n = Elem<T>::from_float(static_cast<float>(v.e[k]) * r);
-      o.e[k] = Elem<T>::from_float(static_cast<float>(n) * static_cast<float>(w.e[k]));
-    }
-    *reinterpret_cast<P *>(out + i) = o;
+    *reinterpret_cast<P *>(out + i) = norm_scale<T, VEC>(v, w, r);
   };
   if constexpr (NV > 0) {
 #pragma unroll
@@ -177,6 +182,146 @@ __global__ __launch_bounds__(kLayerThreads) void silu_mul_kernel(const T *__rest
   *reinterpret_cast<P *>(out + row * width + i) = o;
 }
 
+// ------------------------------------------------- few-token products ---
+//
+// norm_linear_kernel: out = x W^T for up to kLinearRows tokens, x = h or
+// rms_norm(h + y) * weight, out = x W^T or silu(gate) * up of its two halves.
+//
+// What bounds it: a few tokens use each weight once or a few times, so the
+// product streams W; at the sizes of one layer (8-50 MB) a launch's ramp and
+// the latency of that stream count as much as its bytes.  Every wave owns R
+// rows of W (R gate and R up rows), issues its first loads of them before it
+// looks at x, and keeps the next ones in flight; x is staged in LDS by each
+// workgroup for itself, which costs it the norm again (4-8 KB from the L2,
+// while W arrives) and saves the norm's launch.  The dot products run on the
+// VALU with fp32 sums: at this few tokens the matrix cores would wait for W
+// just the same.
+//
+// Measured on MI355X in fp16, one token, against the norm, the library's
+// product and the SwiGLU as launches of their own: 2048 -> 2560 with norm 4.8
+// and 9.8 us, 2048 -> 2 x 5632 with norm and SwiGLU 10.2 and 19.6, 5632 ->
+// 2048 7.3 and 10.4, 4096 -> 2 x 11008 30.4 and 57.1 (5.9 TB/s), 4096 ->
+// 32000 41.3 and 58.3 (6.3 TB/s).  Two tokens take 5-25% longer, the
+// library's no longer; with four, norm and 4096 -> 12288 took 27.9 and
+// 23.8, so the line is at two.
+constexpr int kLinearRows = 2;
+constexpr int64_t kLinearLds = INT64_C(64) << 10;  // x in LDS: two workgroups a CU at least
+
+struct LinearArgs {
+  NormArgs norm;  // h, y, weight (nullptr: x = h), h_out
+  const void *w;  // [n][hidden], or [2 n][hidden] gate then up
+  void *out;      // [rows][n]
+  int32_t n;
+};
+
+template <typename T, int M, int R, bool GLU>
+__global__ __launch_bounds__(kLayerThreads) void norm_linear_kernel(const LinearArgs a) {
+  using E = Elem<T>;
+  constexpr int VEC = 16 / static_cast<int>(sizeof(T));
+  using P = Pack<T, VEC>;
+  constexpr int U = 4, RW = GLU ? 2 * R : R, KSTEP = U * 64 * VEC;
+  extern __shared__ __attribute__((aligned(16))) char s_raw[];
+  __shared__ float s_sum[M][kLayerWaves];
+  T *s_x = reinterpret_cast<T *>(s_raw);  // [rows][K]
+  const int K = a.norm.hidden, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  const int n0 = (static_cast<int>(blockIdx.x) * kLayerWaves + wave) * R;
+
+  // Rows past the last one repeat it (loaded in bounds, not stored).
+  const T *wrow[RW];
+#pragma unroll
+  for (int r = 0; r < RW; ++r) {
+    const int64_t n = min(n0 + r % R, a.n - 1) + (r >= R ? a.n : 0);
+    wrow[r] = static_cast<const T *>(a.w) + n * K + lane * VEC;
+  }
+  using Tile = u32x4[RW][U];
+  auto fetch = [&](int k0, Tile &t) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int k = k0 + u * 64 * VEC;
+        t[r][u] = u32x4{};
+        if (k + lane * VEC < K) t[r][u] = __builtin_nontemporal_load(reinterpret_cast<const u32x4 *>(wrow[r] + k));
+      }
+  };
+  Tile cur;
+  fetch(0, cur);
+
+  const int i0 = static_cast<int>(threadIdx.x) * VEC;
+  for (int m = 0; m < M; ++m) {
+    T *keep = a.norm.h_out && blockIdx.x == 0 ? static_cast<T *>(a.norm.h_out) + m * a.norm.h_out_stride : nullptr;
+    float sum = 0.f;
+    for (int i = i0; i < K; i += kLayerThreads * VEC) {
+      const P v = norm_input<T, VEC>(a.norm, m, i);
+      *reinterpret_cast<P *>(s_x + static_cast<int64_t>(m) * K + i) = v;
+      if (keep) *reinterpret_cast<P *>(keep + i) = v;
+#pragma unroll
+      for (int k = 0; k < VEC; ++k) sum = fmaf(static_cast<float>(v.e[k]), static_cast<float>(v.e[k]), sum);
+    }
+    sum = sum_from<1>(sum);
+    if (lane == 0) s_sum[m][wave] = sum;
+  }
+  __syncthreads();
+  if (a.norm.weight) {
+    for (int m = 0; m < M; ++m) {
+      float total = 0.f;
+#pragma unroll
+      for (int w = 0; w < kLayerWaves; ++w) total += s_sum[m][w];
+      const float r = rsqrtf(total / static_cast<float>(K) + a.norm.eps);
+      for (int i = i0; i < K; i += kLayerThreads * VEC) {
+        P *x = reinterpret_cast<P *>(s_x + static_cast<int64_t>(m) * K + i);
+        *x = norm_scale<T, VEC>(*x, *reinterpret_cast<const P *>(static_cast<const T *>(a.norm.weight) + i), r);
+      }
+    }
+    __syncthreads();
+  }
+
+  float acc[M][RW];
+#pragma unroll
+  for (int m = 0; m < M; ++m)
+#pragma unroll
+    for (int r = 0; r < RW; ++r) acc[m][r] = 0.f;
+  auto consume = [&](int k0, const Tile &t) {
+#pragma unroll
+    for (int u = 0; u < U; ++u) {
+      const int k = k0 + u * 64 * VEC + lane * VEC;
+      if (k >= K) continue;  // its weights are zero
+#pragma unroll
+      for (int m = 0; m < M; ++m) {
+        const u32x4 x = *reinterpret_cast<const u32x4 *>(s_x + static_cast<int64_t>(m) * K + k);
+#pragma unroll
+        for (int r = 0; r < RW; ++r) acc[m][r] = E::dot(x, t[r][u], acc[m][r]);
+      }
+    }
+  };
+  int k0 = 0;
+  for (; k0 + KSTEP < K; k0 += KSTEP) {
+    Tile next;
+    fetch(k0 + KSTEP, next);
+    consume(k0, cur);
+#pragma unroll
+    for (int r = 0; r < RW; ++r)
+#pragma unroll
+      for (int u = 0; u < U; ++u) cur[r][u] = next[r][u];
+  }
+  consume(k0, cur);
+
+#pragma unroll
+  for (int m = 0; m < M; ++m) {
+#pragma unroll
+    for (int r = 0; r < RW; ++r) acc[m][r] = sum_from<1>(acc[m][r]);
+    if (lane == 0) {
+      T *out = static_cast<T *>(a.out) + static_cast<int64_t>(m) * a.n;
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        float v = acc[m][r];
+        if constexpr (GLU) v = v / (1.f + expf(-v)) * acc[m][R + r];
+        if (n0 + r < a.n) out[n0 + r] = E::from_float(v);
+      }
+    }
+  }
+}
+
 // ------------------------------------------------------------------ host ---
 
 static int dtype_size(int dtype, const char *what, int *es) {
@@ -225,7 +370,56 @@ static void launch_silu(const void *gate_up, void *out, bool vec16, int64_t rows
   else silu_mul_kernel<T, 1><<<grid, kLayerThreads, 0, s>>>(static_cast<const T *>(gate_up), static_cast<T *>(out), width);
 }
 
+template <typename T, int M, bool GLU>
+static void launch_linear(const LinearArgs &a, hipStream_t s) {
+  const size_t lds = static_cast<size_t>(M) * a.norm.hidden * sizeof(T);
+  // Two rows a wave once that still gives every CU a workgroup.
+  const int R = a.n >= 2048 ? 2 : 1;
+  const dim3 grid(static_cast<unsigned>((a.n + kLayerWaves * R - 1) / (kLayerWaves * R)));
+  if (R == 2) norm_linear_kernel<T, M, 2, GLU><<<grid, kLayerThreads, lds, s>>>(a);
+  else norm_linear_kernel<T, M, 1, GLU><<<grid, kLayerThreads, lds, s>>>(a);
+}
+
+template <typename T>
+static void dispatch_linear(const LinearArgs &a, int rows, bool glu, hipStream_t s) {
+  static_assert(kLinearRows == 2, "one instance per row count");
+  if (rows == 1) glu ? launch_linear<T, 1, true>(a, s) : launch_linear<T, 1, false>(a, s);
+  else glu ? launch_linear<T, 2, true>(a, s) : launch_linear<T, 2, false>(a, s);
+}
+
 }  // namespace hexkv
+
+extern "C" int hexkv_norm_linear(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
+                                 int64_t h_out_stride, const void *norm_weight, float eps, const void *weight,
+                                 void *out, int rows, int hidden, int n, int glu, int dtype, hexkv_stream_t stream) {
+  using namespace hexkv;
+  clear_error();
+  const char *what = "hexkv_norm_linear";
+  int es = 0;
+  const int rc = dtype_size(dtype, what, &es);
+  if (rc != HEXKV_OK) return rc;
+  if (rows < 0 || hidden < 1 || n < 0 || n > 1 << 28 || h_stride < 0 || y_stride < 0 || h_out_stride < 0)
+    return fail(HEXKV_EINVAL, "%s: bad sizes or a negative stride", what);
+  if (rows == 0 || n == 0) return HEXKV_OK;
+  if (!h || !weight || !out) return fail(HEXKV_EINVAL, "%s: null tensor", what);
+  if (h_out && (h_out == h || h_out == y)) return fail(HEXKV_EINVAL, "%s: h_out must not be h or y", what);
+  const int64_t vec = 16 / es;
+  if (rows > kLinearRows || static_cast<int64_t>(rows) * hidden * es > kLinearLds)
+    return fail(HEXKV_EUNSUPPORTED, "%s: at most %d rows and %lld bytes of them", what, kLinearRows,
+                static_cast<long long>(kLinearLds));
+  if (hidden % vec || h_stride % vec || y_stride % vec || h_out_stride % vec || !aligned16(h) || !aligned16(y) ||
+      !aligned16(h_out) || !aligned16(norm_weight) || !aligned16(weight))
+    return fail(HEXKV_EUNSUPPORTED, "%s: rows must be 16-byte aligned and a multiple of 16 bytes", what);
+  const LinearArgs a{NormArgs{h, y, norm_weight, h_out, nullptr, h_stride, y_stride, h_out_stride, hidden, eps},
+                     weight, out, n};
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  switch (dtype) {
+    case HEXKV_BF16: dispatch_linear<__bf16>(a, rows, glu != 0, s); break;
+    case HEXKV_F16: dispatch_linear<_Float16>(a, rows, glu != 0, s); break;
+    default: dispatch_linear<float>(a, rows, glu != 0, s); break;
+  }
+  return check_launch(what);
+}
 
 extern "C" int hexkv_add_rms_norm(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
                                   int64_t h_out_stride, const void *weight, void *out, int64_t rows, int hidden,

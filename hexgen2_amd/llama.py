@@ -115,6 +115,20 @@ class LlamaHost:
             state.update(values)
         return cls(shape, state, device, dtype)
 
+    def _norm_linear(self, h, y, norm, weight, glu=False, keep_sum=True):
+        """``(product, h + y)`` of RMSNorm(h + y) and ``weight``, with ``glu``
+        SwiGLU of its two halves: one launch for a few tokens, else the norm's,
+        the library product and the SwiGLU's."""
+        if ops.linear_fits(h, norm, weight):
+            return ops.norm_linear(h, y, norm, self.shape.rms_norm_eps, weight, glu, keep_sum)
+        x = F.linear(ops.add_rms_norm(h, y, norm, self.shape.rms_norm_eps, keep_sum), weight)
+        return (ops.silu_mul(x) if glu else x), h
+
+    def _linear(self, x, weight):
+        if ops.linear_fits(x, weight):
+            return ops.norm_linear(x, None, None, 0.0, weight)[0]
+        return F.linear(x, weight)
+
     @torch.inference_mode()
     def forward(self, input_ids: torch.Tensor, inference_params, last_token_only: bool = True,
                 fused_append: bool = False) -> torch.Tensor:
@@ -132,8 +146,7 @@ class LlamaHost:
         h = F.embedding(input_ids, self.embed)
         y = None  # the block output still to be added to h
         for i, layer in enumerate(self.layers):
-            x = ops.add_rms_norm(h, y, layer["ln1"], s.rms_norm_eps)
-            qkv = F.linear(x, layer["wqkv"])
+            qkv, h = self._norm_linear(h, y, layer["ln1"], layer["wqkv"])
             if inference_params.fused_ft_kernel and offset > 0:
                 # FT decode (mha.py:553-571): rotary, append and attention in one call
                 q = qkv[..., :heads * d].view(batch, seqlen, heads, d)
@@ -147,9 +160,9 @@ class LlamaHost:
                     kv_view = _update_kv_cache(kv, inference_params, i)
                     # prompt (offset 0): causal; decode: causal=False (mha.py:566-569)
                     context = self.attn(q, kv_view, causal=None if offset == 0 else False)
-            y = F.linear(context.reshape(batch, seqlen, -1), layer["wo"])
-            x = ops.add_rms_norm(h, y, layer["ln2"], s.rms_norm_eps)
-            y = F.linear(ops.silu_mul(F.linear(x, layer["gate_up"])), layer["down"])
+            y = self._linear(context.reshape(batch, seqlen, -1), layer["wo"])
+            x, h = self._norm_linear(h, y, layer["ln2"], layer["gate_up"], glu=True)
+            y = self._linear(x, layer["down"])
         if last_token_only:
             h, y = h[:, -1], None if y is None else y[:, -1]
-        return F.linear(ops.add_rms_norm(h, y, self.norm, s.rms_norm_eps, keep_sum=False), self.lm_head)
+        return self._norm_linear(h, y, self.norm, self.lm_head, keep_sum=False)[0]

@@ -729,6 +729,56 @@ def add_rms_norm(h: torch.Tensor, y: Optional[torch.Tensor], weight: torch.Tenso
     return out
 
 
+LINEAR_ROWS, LINEAR_BYTES = 2, 64 << 10  # tokens hexkv_norm_linear takes, and their bytes
+
+
+def linear_fits(x: torch.Tensor, *weights: torch.Tensor) -> bool:
+    """Whether ``norm_linear`` takes tokens ``x [..., hidden]`` (rows at one
+    stride) with these contiguous weights ``[n, hidden]``: up to 2 tokens of
+    at most 64 KB, everything 16-byte aligned."""
+    hidden, elem = x.shape[-1], x.element_size()
+    rows = x.numel() // hidden if hidden else 0
+    return (0 < rows <= LINEAR_ROWS and rows * hidden * elem <= LINEAR_BYTES and hidden * elem % 16 == 0
+            and x.dtype in _DTYPES and x.data_ptr() % 16 == 0
+            and all(w.is_contiguous() and w.data_ptr() % 16 == 0 and w.dtype == x.dtype for w in weights))
+
+
+def norm_linear(h: torch.Tensor, y: Optional[torch.Tensor], norm_weight: Optional[torch.Tensor], eps: float,
+                weight: torch.Tensor, glu: bool = False, keep_sum: bool = True):
+    """``(out, sum)`` of up to 2 tokens in one launch: ``sum = h + y`` (``h``
+    itself without ``y``, not formed without ``keep_sum``), ``out =
+    rms_norm(sum) * norm_weight @ weight.T`` (``norm_weight`` None: ``h @
+    weight.T``), with ``glu`` ``silu(gate) * up`` of ``weight``'s two halves."""
+    _require_device(h, weight)
+    hidden = h.shape[-1]
+    if h.dtype not in _DTYPES or weight.dtype != h.dtype or weight.device != h.device:
+        raise ValueError("h and weight must share one of float16, bfloat16, float32 and a device")
+    if weight.dim() != 2 or weight.shape[1] != hidden or not weight.is_contiguous() or (glu and weight.shape[0] % 2):
+        raise ValueError(f"weight must be contiguous [n, {hidden}], got {tuple(weight.shape)}")
+    norm_ptr = y_ptr = kept = None
+    y_stride = 0
+    total = h
+    if norm_weight is not None:
+        if norm_weight.shape != (hidden,) or norm_weight.dtype != h.dtype or norm_weight.device != h.device \
+                or not norm_weight.is_contiguous():
+            raise ValueError(f"norm_weight must be contiguous [{hidden}] like h, got {tuple(norm_weight.shape)}")
+        norm_ptr = norm_weight.data_ptr()
+    if y is not None:
+        if norm_weight is None or y.shape != h.shape or y.dtype != h.dtype or y.device != h.device:
+            raise ValueError("y goes with norm_weight, and must share h's shape, dtype and device")
+        y_ptr, y_stride = y.data_ptr(), _row_stride(y, "y")
+        if keep_sum:
+            total = h.new_empty(h.shape)
+            kept = total.data_ptr()
+    n = weight.shape[0] // 2 if glu else weight.shape[0]
+    out = h.new_empty((*h.shape[:-1], n))
+    rc = _lib.load().hexkv_norm_linear(h.data_ptr(), _row_stride(h, "h"), y_ptr, y_stride, kept, hidden, norm_ptr, eps,
+                                       weight.data_ptr(), out.data_ptr(), h.numel() // hidden if hidden else 0, hidden,
+                                       n, 1 if glu else 0, _DTYPES[h.dtype], _stream(h))
+    _lib.check(rc, "hexkv_norm_linear")
+    return out, total
+
+
 def _row_stride(t: torch.Tensor, name: str) -> int:
     """Elements between consecutive rows (last dim) of ``t``, whose outer
     dims must fold into one."""

@@ -614,6 +614,16 @@ int hexkv_add_rms_norm(const void *h, int64_t h_stride, const void *y, int64_t y
                        int64_t h_out_stride, const void *weight, void *out, int64_t rows, int hidden,
                        float eps, int dtype, hexkv_stream_t stream);
 
+/* out = x W^T for up to 2 tokens, W [n][hidden] (contiguous), one launch:
+ * x = h, or with norm_weight rms_norm(h + y) * norm_weight (y may be NULL),
+ * the sum also written to h_out (NULL, or neither h nor y).  With glu W is
+ * [2 n][hidden] and out[i] = silu(x W[i]) * (x W[n + i]), rounded once.
+ * HEXKV_EUNSUPPORTED above 2 rows or 64 KiB of them, or when hidden, strides
+ * or addresses are not multiples of 16 bytes. */
+int hexkv_norm_linear(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
+                      int64_t h_out_stride, const void *norm_weight, float eps, const void *weight,
+                      void *out, int rows, int hidden, int n, int glu, int dtype, hexkv_stream_t stream);
+
 /* Rows [q heads | k heads | v heads] of head_dim elements (qkv_stride apart)
  * into q [rows][q_heads][head_dim] and kv [rows][2][kv_heads][head_dim], q
  * and k rotated (GPT-NeoX halves) by position * inv_freq_dev[j].  Row r is

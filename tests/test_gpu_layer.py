@@ -75,6 +75,58 @@ def test_silu_mul(dtype, width):
     _within(ops.silu_mul(gate_up), want, (UNIT[dtype] * 1.01 + FP32) * want.abs() + TINY)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("rows", [1, 2])
+@pytest.mark.parametrize("hidden,n", [(8, 1), (64, 7), (504, 1023), (512, 2047), (520, 2048), (2048, 2050), (4104, 9),
+                                      (5632, 64), (8192, 33)])
+def test_norm_linear(dtype, rows, hidden, n):
+    """Each lane sums hidden / 64 products in fp32, then six levels of a tree."""
+    torch.manual_seed(hidden + n)
+    h, y = (torch.randn(rows, 1, hidden, device="cuda").to(dtype) for _ in range(2))
+    norm = torch.randn(hidden, device="cuda").to(dtype)
+    w = (torch.randn(2 * n, hidden, device="cuda") * hidden ** -0.5).to(dtype)
+    total = h.clone()
+    x = ops.add_rms_norm(total, y, norm, 1e-5)  # the same roundings
+    steps = (hidden + 63) // 64 + 8
+
+    def product(x, w):
+        return x.double() @ w.double().T, steps * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T)
+
+    want, err = product(h, w[:n])
+    got, same = ops.norm_linear(h, None, None, 0.0, w[:n].contiguous())
+    assert same is h
+    _within(got, want, 1.01 * UNIT[dtype] * want.abs() + err + TINY)
+    # the norm's own sum may round one value of x the other way
+    flip = 2 * UNIT[dtype] * (x.double().abs().amax(-1, keepdim=True) * w.double().abs().amax())
+    want, err = product(x, w[:n])
+    got, kept = ops.norm_linear(h, y, norm, 1e-5, w[:n].contiguous())
+    assert torch.equal(kept, total) and not torch.equal(kept, h)
+    _within(got, want, 1.01 * UNIT[dtype] * want.abs() + err + 8 * flip + TINY)
+    both, err = product(x, w)
+    g, u = both[..., :n], both[..., n:]
+    silu = g * torch.sigmoid(g)
+    eg, eu = (err + 8 * flip)[..., :n], (err + 8 * flip)[..., n:]
+    got, kept = ops.norm_linear(h, y, norm, 1e-5, w, glu=True, keep_sum=False)
+    assert kept is h
+    bound = (1.01 * UNIT[dtype] + FP32) * (silu * u).abs() + 1.1 * u.abs() * eg + silu.abs() * eu + 1.1 * eg * eu
+    _within(got, silu * u, bound + TINY)
+
+
+def test_norm_linear_fits_and_refuses():
+    x, w = torch.zeros(2, 1, 64, device="cuda").half(), torch.zeros(16, 64, device="cuda").half()
+    assert ops.linear_fits(x, w)
+    wide = torch.zeros(1, 1, 32776, device="cuda").half()
+    for bad in (torch.zeros(3, 1, 64, device="cuda").half(), wide, x[..., :60], x[:0], x.double()):
+        assert not ops.linear_fits(bad, w)
+    assert not ops.linear_fits(x, w.T) and not ops.linear_fits(x, w.float())
+    with pytest.raises(NotImplementedError):
+        ops.norm_linear(wide, None, None, 0.0, torch.zeros(1, 32776, device="cuda").half())
+    with pytest.raises(ValueError):
+        ops.norm_linear(x, x, None, 0.0, w)
+    with pytest.raises(ValueError):
+        ops.norm_linear(x, None, None, 0.0, w[:, :32])
+
+
 def test_layer_steps_refuse_what_they_cannot_address():
     x = torch.zeros(2, 3, 8, device="cuda", dtype=torch.float16)
     w = torch.zeros(8, device="cuda", dtype=torch.float16)
