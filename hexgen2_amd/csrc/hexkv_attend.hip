@@ -479,28 +479,36 @@ __device__ __forceinline__ u32x4 pack16(const float *f) {
 // and its sine and cosine are evaluated in fp64 (an fp32 angle is off by
 // ~pos * 2^-24 radians, 6e-5 at position 1000); the turn itself is fp32.
 // The caller rounds both back to T when it packs them, as the reference
-// kernel does.
+// kernel does.  A pair's sine and cosine are the same for every head:
+// rot_dim / 2 lanes evaluate them once per workgroup (s_rot), since with
+// several rounds of workgroups the fp64 work of every lane for every head
+// held up the stream.
 template <typename T, int D, int G>
-__device__ __forceinline__ void ft_prologue(const AttendArgs &a, const Work &w, float *sq, float *skn) {
+__device__ __forceinline__ void ft_prologue(const AttendArgs &a, const Work &w, float *sq, float *skn, float2 *s_rot) {
   const T *q = static_cast<const T *>(a.q) + w.b * a.q_bs + w.qh0 * D;
   for (int i = threadIdx.x; i < G * D; i += kAttThreads) sq[i] = static_cast<float>(q[i]);
   if (w.has_new) {
     const T *k = static_cast<const T *>(a.kv_new) + w.b * a.new_bs + static_cast<int64_t>(w.hk) * D;
     for (int i = threadIdx.x; i < D; i += kAttThreads) skn[i] = static_cast<float>(k[i]);
   }
-  __syncthreads();
   const int half = a.rot_dim / 2;
+  static_assert(D / 2 <= kAttThreads, "one lane per pair");
+  if (static_cast<int>(threadIdx.x) < half) {
+    const int j = threadIdx.x;
+    const double theta =
+        static_cast<double>(w.pos_new) * exp2(-static_cast<double>(2 * j) / a.rot_dim * a.rot_log2_base);
+    double sd, cd;
+    sincos(theta, &sd, &cd);
+    s_rot[j] = float2{static_cast<float>(cd), static_cast<float>(sd)};
+  }
+  __syncthreads();
   if (half > 0) {
-    const int pos = w.pos_new;
     const int vecs = w.has_new ? G + 1 : G;
     for (int i = threadIdx.x; i < vecs * half; i += kAttThreads) {
       const int g = i / half, j = i - g * half;
       float *x = g < G ? sq + g * D : skn;
       const int i0 = a.rot_neox ? j : 2 * j, i1 = a.rot_neox ? j + half : 2 * j + 1;
-      const double theta = static_cast<double>(pos) * exp2(-static_cast<double>(2 * j) / a.rot_dim * a.rot_log2_base);
-      double sd, cd;
-      sincos(theta, &sd, &cd);
-      const float sn = static_cast<float>(sd), cs = static_cast<float>(cd);
+      const float cs = s_rot[j].x, sn = s_rot[j].y;
       const float x0 = x[i0], x1 = x[i1];
       x[i0] = x0 * cs - x1 * sn;
       x[i1] = x0 * sn + x1 * cs;
@@ -520,6 +528,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
   __shared__ __attribute__((aligned(16))) float s_acc[kAttWaves][G][D];
   __shared__ float s_m[kAttWaves][G], s_l[kAttWaves][G];
   __shared__ float s_kn[FT ? D : 1];
+  __shared__ float2 s_rot[FT ? D / 2 : 1];
   // FT: two staged K tiles, STEP positions of D / VEC 16-byte chunks each,
   // one padded row per position.
   constexpr int KT_PITCH = D / VEC * 16 + 16;
@@ -532,15 +541,8 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
   const int sub = lane % LPP, gid = wave * GPW + lane / LPP;
   const float scale = a.scale_log2;
 
-  u32x4 qv[G][NV];
-  if constexpr (FT) {
-    ft_prologue<T, D, G>(a, w, &s_acc[0][0][0], s_kn);
-#pragma unroll
-    for (int g = 0; g < G; ++g)
-#pragma unroll
-      for (int v = 0; v < NV; ++v) qv[g][v] = pack16<T>(&s_acc[0][g][sub * EPL + v * VEC]);
-    __syncthreads();  // every wave holds its query before s_acc is written again
-  } else {
+  u32x4 qv[G][NV];  // FT: rotated and packed below, with the first tile in flight
+  if constexpr (!FT) {
     const T *qrow = static_cast<const T *>(a.q) + w.b * a.q_bs + w.t * a.q_rs + w.qh0 * D + sub * EPL;
 #pragma unroll
     for (int g = 0; g < G; ++g)
@@ -698,11 +700,19 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
                                                       (sub * NV + v) * 16);
     };
     const int nfull = w.n_cache / STEP, ntiles = (w.n_cache + STEP - 1) / STEP;
+    u32x4 kt[CPT];
+    Slots vr;
     if (ntiles > 0) {
-      u32x4 kt[CPT];
-      Slots vr;
       kt_fetch(0, kt);
       v_fetch(0, vr);
+    }
+    ft_prologue<T, D, G>(a, w, &s_acc[0][0][0], s_kn, s_rot);
+#pragma unroll
+    for (int g = 0; g < G; ++g)
+#pragma unroll
+      for (int v = 0; v < NV; ++v) qv[g][v] = pack16<T>(&s_acc[0][g][sub * EPL + v * VEC]);
+    __syncthreads();  // every wave holds its query before s_acc is written again
+    if (ntiles > 0) {
       kt_store(0, kt);
       __syncthreads();
       for (int t = 0; t < nfull; ++t) {
@@ -1531,14 +1541,33 @@ static int segment_heads(const hexkv_attend_params *p) {
 // measured slower on every one of these shapes (Llama-3-8B 172.5 vs 171.1 us,
 // the 70B TP-8 share 26.3 vs 15.9): at 512 positions the partitions already
 // balance the launch, and finer pieces only add partials to merge.
-static int choose_partition(const hexkv_attend_params *p) {
-  if (p->partition > 0) return p->partition;
+static int64_t wanted_partition(const hexkv_attend_params *p) {
   const int64_t rows = static_cast<int64_t>(p->batch) * p->q_len;
   const int64_t groups = p->q_heads / kernel_group(p->q_heads / p->kv_heads);
   const int64_t half = std::max<int64_t>(1, (p->max_seqlen + 1) / 2);
-  const int64_t want = rows * groups * half / 2048;
+  return rows * groups * half / 2048;
+}
+
+static int base_partition(const hexkv_attend_params *p) {
+  if (p->partition > 0) return p->partition;
+  const int64_t want = wanted_partition(p);
   int part = 128;
   while (part < 512 && part < want) part <<= 1;
+  return part;
+}
+
+// Decode rows take 192 positions instead of 128 where the call is large
+// enough to fill the chip with them and its rows are long (a 128-position
+// stride also puts one index of every row on the same memory channels).
+// Measured per call with the merge, 192 and 128: Llama-2-7B 1 x 8192 28.4
+// and 39.1 us, 8 x 2048 46.5 and 54.0, 8 x 256-2048 25.5 and 26.9;
+// Llama-3-8B 16 x 128-2048 23.1 and 24.9, 1 x 8192 14.4 and 16.1; TinyLlama
+// 32 x 512-4096 25.0 and 27.6.  Below a want of 16 or 1024 positions 128
+// leads (Llama-2-7B 4 x 100-700: 10.4 and 10.9; TinyLlama 1 x 2048: 6.6 and
+// 7.3).
+static int choose_partition(const hexkv_attend_params *p) {
+  const int part = base_partition(p);
+  if (p->partition == 0 && p->q_len == 1 && part == 128 && p->max_seqlen > 1024 && wanted_partition(p) >= 16) return 192;
   return part;
 }
 
@@ -1554,7 +1583,7 @@ static bool use_tiles(const hexkv_attend_params *p) {
 // below the per-row kernels' partition, so no call needs more workspace
 // than it did with one.
 static int tile_partition(const hexkv_attend_params *p) {
-  const int per_row = choose_partition(p);
+  const int per_row = base_partition(p);
   if (p->partition > 0) return per_row;
   const int64_t rows = static_cast<int64_t>(p->q_len) * (p->q_heads / p->kv_heads);
   const int64_t per = tile_rows(rows);
@@ -1562,6 +1591,13 @@ static int tile_partition(const hexkv_attend_params *p) {
   const int64_t parts = std::max<int64_t>(1, 512 / std::max<int64_t>(1, tiles));
   const int64_t part = (std::max<int64_t>(p->max_seqlen, 1) + parts * 64 - 1) / (parts * 64) * 64;
   return static_cast<int>(std::max<int64_t>(part, per_row));
+}
+
+// The partition whose need the size queries report: never above the one a
+// call runs with, so a workspace sized for the longest step of a loop (and a
+// saved size) serves its shorter ones wherever choose_partition's lines lie.
+static int sizing_partition(const hexkv_attend_params *p) {
+  return use_tiles(p) ? tile_partition(p) : base_partition(p);
 }
 
 static int partition_of(const hexkv_attend_params *p) {
@@ -2154,7 +2190,7 @@ extern "C" size_t hexkv_attend_workspace_bytes(const hexkv_attend_params *p) {
   if (!p || p->q_heads < 1 || p->kv_heads < 1 || p->q_heads % p->kv_heads || p->q_len < 1 ||
       p->batch < 0 || p->max_seqlen < 0)
     return 0;
-  return workspace_bytes(p, partition_of(p));
+  return workspace_bytes(p, sizing_partition(p));
 }
 
 extern "C" int hexkv_attend_kernel(const hexkv_attend_params *p) {
@@ -2480,9 +2516,9 @@ extern "C" int hexkv_attend_noalloc(const hexkv_attend_params *p, hexkv_stream_t
   const char *what = "hexkv_attend_noalloc";
   int rc = validate(p);
   if (rc != HEXKV_OK || p->batch == 0) return rc;
-  // The limit is the per-row kernels' need, whichever kernel runs (the tile
-  // kernel never needs more), so it does not depend on the kernel choice.
-  const size_t limit_need = workspace_bytes(p, choose_partition(p));
+  // The limit is the need at the base partition, whichever kernel and
+  // partition run (none needs more), so it does not move with their rules.
+  const size_t limit_need = workspace_bytes(p, base_partition(p));
   if (limit_need > HEXKV_NOALLOC_SCRATCH_BYTES)
     return fail(HEXKV_EWORKSPACE,
                 "%s: this call needs %zu bytes of split-K workspace, above the %u-byte static scratch "
@@ -2563,7 +2599,7 @@ extern "C" size_t hexkv_ft_attend_workspace_bytes(const hexkv_ft_attend_params *
       p->max_position < 0)
     return 0;
   const hexkv_attend_params g = ft_geometry(p);
-  return workspace_bytes(&g, choose_partition(&g));
+  return workspace_bytes(&g, base_partition(&g));
 }
 
 extern "C" int hexkv_ft_attend(const hexkv_ft_attend_params *p, void *workspace, size_t ws_bytes,

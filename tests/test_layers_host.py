@@ -70,3 +70,20 @@ def test_layers_independent(change, free):
     elif change == "lengths":
         p.lengths_out_dev = a.out + 8
     assert lib.hexkv_attend_layers_independent(p, (_lib.AttendLayer * 2)(a, b), 2) == free
+
+
+@pytest.mark.parametrize("dtype,hq,hkv,d", [(0, 32, 4, 64), (0, 32, 32, 128), (1, 8, 1, 128), (1, 32, 8, 128)])
+@pytest.mark.parametrize("batch", [1, 8, 64])
+def test_workspace_sizes_follow_the_base_partition(dtype, hq, hkv, d, batch):
+    """A decode loop's workspace, sized for its longest step, covers the
+    shorter ones up to where the 128-position rule itself doubles."""
+    lib = _lib.load()
+    group = next(g for g in (8, 4, 2, 1) if (hq // hkv) % g == 0)
+    for longest in (129, 1024, 1025, 1100, 2048, 4096):
+        want = batch * (hq // group) * ((longest + 1) // 2) // 2048
+        part = next((p for p in (128, 256) if p >= want), 512)
+        parts = (longest + part - 1) // part
+        p = _lib.AttendParams(dtype=dtype, batch=batch, q_len=1, q_heads=hq, kv_heads=hkv, head_dim=d, softmax_scale=1.0,
+                              capacity=longest, max_seqlen=longest)
+        need = _lib.ATTEND_COUNTER_BYTES + batch * hq * parts * (d + 2) * 4 if parts > 1 else 0
+        assert lib.hexkv_attend_workspace_bytes(p) == need
