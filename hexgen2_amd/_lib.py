@@ -23,7 +23,7 @@ EXPORTS = ("hexkv_version", "hexkv_last_error", "hexkv_pack", "hexkv_unpack", "h
            "hexkv_head_concat", "hexkv_ipc_export", "hexkv_ipc_open", "hexkv_ipc_close",
            "hexkv_ipc_dlpack", "hexkv_ft_store", "hexkv_ft_attend_workspace_bytes", "hexkv_ft_attend",
            "hexkv_attend_noalloc", "hexkv_attend_plan", "hexkv_attend_plan_chunk", "hexkv_attend_plan_kernel",
-           "hexkv_device_status", "hexkv_device_xcds", "hexkv_add_rms_norm", "hexkv_rope_split", "hexkv_silu_mul", "hexkv_norm_linear",
+           "hexkv_device_status", "hexkv_device_xcds", "hexkv_add_rms_norm", "hexkv_rope_split", "hexkv_silu_mul", "hexkv_norm_linear", "hexkv_norm_rope_linear",
            "hexkv_attend_layers", "hexkv_attend_layers_workspace_bytes", "hexkv_attend_layers_independent",
            "hexkv_attend_plan_layers")
 NOALLOC_SCRATCH_BYTES = 32 << 20
@@ -176,6 +176,9 @@ def load() -> ctypes.CDLL:
     lib.hexkv_add_rms_norm.argtypes = [vp, i64, vp, i64, vp, i64, vp, vp, i64, ci, ctypes.c_float, ci, vp]
     lib.hexkv_norm_linear.restype = ci
     lib.hexkv_norm_linear.argtypes = [vp, i64, vp, i64, vp, i64, vp, ctypes.c_float, vp, vp, ci, ci, ci, ci, ci, vp]
+    lib.hexkv_norm_rope_linear.restype = ci
+    lib.hexkv_norm_rope_linear.argtypes = [vp, i64, vp, i64, vp, i64, vp, ctypes.c_float, vp, vp, vp, ci, vp, vp,
+                                           ci, ci, ci, ci, ci, ci, ci, vp]
     lib.hexkv_rope_split.restype = ci
     lib.hexkv_rope_split.argtypes = [vp, i64, vp, vp, ci, vp, vp, i64, ci, ci, ci, ci, ci, vp]
     lib.hexkv_silu_mul.restype = ci

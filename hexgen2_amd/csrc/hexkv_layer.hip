@@ -8,7 +8,8 @@
 // memory: every element is read once and written once, in 16-byte vectors.
 // Measured on MI355X with a 4-layer model of TinyLlama's width (512-token
 // prompt, handoff and three decode steps; q/k/v and gate/up each one product
-// as well): 7.33 ms as separate operations, 2.52 ms with these kernels.
+// as well): 7.33 ms as separate operations, 2.52 ms with the three above the
+// few-token products.
 //
 // Each row is one token; a workgroup takes a row (a piece of it where a row
 // is long), so a one-token step still has its row spread over 256 lanes.
@@ -201,7 +202,8 @@ __global__ __launch_bounds__(kLayerThreads) void silu_mul_kernel(const T *__rest
 // product and the SwiGLU as launches of their own: 2048 -> 2560 with norm 4.8
 // and 9.8 us, 2048 -> 2 x 5632 with norm and SwiGLU 10.2 and 19.6, 5632 ->
 // 2048 7.3 and 10.4, 4096 -> 2 x 11008 30.4 and 57.1 (5.9 TB/s), 4096 ->
-// 32000 41.3 and 58.3 (6.3 TB/s).  Two tokens take 5-25% longer, the
+// 32000 41.3 and 58.3 (6.3 TB/s); with the heads split and turned in it as
+// well the model call of the head comment goes from 1.48 to 1.41 ms.  Two tokens take 5-25% longer, the
 // library's no longer; with four, norm and 4096 -> 12288 took 27.9 and
 // 23.8, so the line is at two.
 constexpr int kLinearRows = 2;
@@ -212,14 +214,22 @@ struct LinearArgs {
   const void *w;  // [n][hidden], or [2 n][hidden] gate then up
   void *out;      // [rows][n]
   int32_t n;
+  RopeArgs rope;  // kLinearRope: w is the q, k and v heads, n their pairs of dimensions
 };
 
-template <typename T, int M, int R, bool GLU>
+// What becomes of the two rows of W that a wave takes together.
+enum LinearKind {
+  kLinearPlain,  // one row: its product
+  kLinearGlu,    // gate i, up i: silu(gate) * up
+  kLinearRope,   // dimensions j and j + D / 2 of a head: turned (q, k) or not (v)
+};
+
+template <typename T, int M, int R, int KIND>
 __global__ __launch_bounds__(kLayerThreads) void norm_linear_kernel(const LinearArgs a) {
   using E = Elem<T>;
   constexpr int VEC = 16 / static_cast<int>(sizeof(T));
   using P = Pack<T, VEC>;
-  constexpr int U = 4, RW = GLU ? 2 * R : R, KSTEP = U * 64 * VEC;
+  constexpr int U = 4, RW = KIND == kLinearPlain ? R : 2 * R, KSTEP = U * 64 * VEC;
   extern __shared__ __attribute__((aligned(16))) char s_raw[];
   __shared__ float s_sum[M][kLayerWaves];
   T *s_x = reinterpret_cast<T *>(s_raw);  // [rows][K]
@@ -230,7 +240,13 @@ __global__ __launch_bounds__(kLayerThreads) void norm_linear_kernel(const Linear
   const T *wrow[RW];
 #pragma unroll
   for (int r = 0; r < RW; ++r) {
-    const int64_t n = min(n0 + r % R, a.n - 1) + (r >= R ? a.n : 0);
+    int64_t n = min(n0 + r % R, a.n - 1);
+    if constexpr (KIND == kLinearRope) {
+      const int half = a.rope.head_dim / 2;
+      n += n / half * half + (r >= R ? half : 0);
+    } else {
+      n += r >= R ? a.n : 0;
+    }
     wrow[r] = static_cast<const T *>(a.w) + n * K + lane * VEC;
   }
   using Tile = u32x4[RW][U];
@@ -310,12 +326,35 @@ __global__ __launch_bounds__(kLayerThreads) void norm_linear_kernel(const Linear
   for (int m = 0; m < M; ++m) {
 #pragma unroll
     for (int r = 0; r < RW; ++r) acc[m][r] = sum_from<1>(acc[m][r]);
-    if (lane == 0) {
+    if (lane != 0) continue;
+    if constexpr (KIND == kLinearRope) {
+      const RopeArgs &p = a.rope;
+      const int half = p.head_dim / 2, b = m / p.seqlen;
+      const float pos = static_cast<float>(p.positions ? p.positions[b] : p.offset + m - b * p.seqlen);
+#pragma unroll
+      for (int r = 0; r < R; ++r) {
+        if (n0 + r >= a.n) continue;
+        const int head = (n0 + r) / half, j = n0 + r - head * half;
+        float x0 = acc[m][r], x1 = acc[m][R + r];
+        if (head < p.q_heads + p.kv_heads) {
+          float sn, cs;
+          sincosf(pos * p.inv_freq[j], &sn, &cs);
+          const float u = x0, v = x1;
+          x0 = u * cs - v * sn;
+          x1 = v * cs + u * sn;
+        }
+        T *dst = head < p.q_heads
+                     ? static_cast<T *>(p.q) + (static_cast<int64_t>(m) * p.q_heads + head) * p.head_dim
+                     : static_cast<T *>(p.kv) + (static_cast<int64_t>(m) * 2 * p.kv_heads + head - p.q_heads) * p.head_dim;
+        dst[j] = E::from_float(x0);
+        dst[j + half] = E::from_float(x1);
+      }
+    } else {
       T *out = static_cast<T *>(a.out) + static_cast<int64_t>(m) * a.n;
 #pragma unroll
       for (int r = 0; r < R; ++r) {
         float v = acc[m][r];
-        if constexpr (GLU) v = v / (1.f + expf(-v)) * acc[m][R + r];
+        if constexpr (KIND == kLinearGlu) v = v / (1.f + expf(-v)) * acc[m][R + r];
         if (n0 + r < a.n) out[n0 + r] = E::from_float(v);
       }
     }
@@ -370,21 +409,44 @@ static void launch_silu(const void *gate_up, void *out, bool vec16, int64_t rows
   else silu_mul_kernel<T, 1><<<grid, kLayerThreads, 0, s>>>(static_cast<const T *>(gate_up), static_cast<T *>(out), width);
 }
 
-template <typename T, int M, bool GLU>
+template <typename T, int M, int KIND>
 static void launch_linear(const LinearArgs &a, hipStream_t s) {
   const size_t lds = static_cast<size_t>(M) * a.norm.hidden * sizeof(T);
-  // Two rows a wave once that still gives every CU a workgroup.
+  // Two rows (or pairs) a wave once that still gives every CU a workgroup.
   const int R = a.n >= 2048 ? 2 : 1;
   const dim3 grid(static_cast<unsigned>((a.n + kLayerWaves * R - 1) / (kLayerWaves * R)));
-  if (R == 2) norm_linear_kernel<T, M, 2, GLU><<<grid, kLayerThreads, lds, s>>>(a);
-  else norm_linear_kernel<T, M, 1, GLU><<<grid, kLayerThreads, lds, s>>>(a);
+  if (R == 2) norm_linear_kernel<T, M, 2, KIND><<<grid, kLayerThreads, lds, s>>>(a);
+  else norm_linear_kernel<T, M, 1, KIND><<<grid, kLayerThreads, lds, s>>>(a);
 }
 
-template <typename T>
-static void dispatch_linear(const LinearArgs &a, int rows, bool glu, hipStream_t s) {
+template <typename T, int KIND>
+static void dispatch_rows_of(const LinearArgs &a, int rows, hipStream_t s) {
   static_assert(kLinearRows == 2, "one instance per row count");
-  if (rows == 1) glu ? launch_linear<T, 1, true>(a, s) : launch_linear<T, 1, false>(a, s);
-  else glu ? launch_linear<T, 2, true>(a, s) : launch_linear<T, 2, false>(a, s);
+  if (rows == 1) launch_linear<T, 1, KIND>(a, s);
+  else launch_linear<T, 2, KIND>(a, s);
+}
+
+template <int KIND>
+static void dispatch_linear(const LinearArgs &a, int rows, int dtype, hipStream_t s) {
+  switch (dtype) {
+    case HEXKV_BF16: dispatch_rows_of<__bf16, KIND>(a, rows, s); break;
+    case HEXKV_F16: dispatch_rows_of<_Float16, KIND>(a, rows, s); break;
+    default: dispatch_rows_of<float, KIND>(a, rows, s); break;
+  }
+}
+
+// The checks that every norm_linear_kernel launch shares.
+static int check_linear(const NormArgs &a, const void *weight, int rows, int es, const char *what) {
+  if (a.h_out && (a.h_out == a.h || a.h_out == a.y)) return fail(HEXKV_EINVAL, "%s: h_out must not be h or y", what);
+  if (a.h_stride < 0 || a.y_stride < 0 || a.h_out_stride < 0) return fail(HEXKV_EINVAL, "%s: negative stride", what);
+  const int64_t vec = 16 / es;
+  if (rows > kLinearRows || static_cast<int64_t>(rows) * a.hidden * es > kLinearLds)
+    return fail(HEXKV_EUNSUPPORTED, "%s: at most %d rows and %lld bytes of them", what, kLinearRows,
+                static_cast<long long>(kLinearLds));
+  if (a.hidden % vec || a.h_stride % vec || a.y_stride % vec || a.h_out_stride % vec || !aligned16(a.h) ||
+      !aligned16(a.y) || !aligned16(a.h_out) || !aligned16(a.weight) || !aligned16(weight))
+    return fail(HEXKV_EUNSUPPORTED, "%s: rows must be 16-byte aligned and a multiple of 16 bytes", what);
+  return HEXKV_OK;
 }
 
 }  // namespace hexkv
@@ -398,26 +460,44 @@ extern "C" int hexkv_norm_linear(const void *h, int64_t h_stride, const void *y,
   int es = 0;
   const int rc = dtype_size(dtype, what, &es);
   if (rc != HEXKV_OK) return rc;
-  if (rows < 0 || hidden < 1 || n < 0 || n > 1 << 28 || h_stride < 0 || y_stride < 0 || h_out_stride < 0)
-    return fail(HEXKV_EINVAL, "%s: bad sizes or a negative stride", what);
+  if (rows < 0 || hidden < 1 || n < 0 || n > 1 << 28) return fail(HEXKV_EINVAL, "%s: bad sizes", what);
   if (rows == 0 || n == 0) return HEXKV_OK;
   if (!h || !weight || !out) return fail(HEXKV_EINVAL, "%s: null tensor", what);
-  if (h_out && (h_out == h || h_out == y)) return fail(HEXKV_EINVAL, "%s: h_out must not be h or y", what);
-  const int64_t vec = 16 / es;
-  if (rows > kLinearRows || static_cast<int64_t>(rows) * hidden * es > kLinearLds)
-    return fail(HEXKV_EUNSUPPORTED, "%s: at most %d rows and %lld bytes of them", what, kLinearRows,
-                static_cast<long long>(kLinearLds));
-  if (hidden % vec || h_stride % vec || y_stride % vec || h_out_stride % vec || !aligned16(h) || !aligned16(y) ||
-      !aligned16(h_out) || !aligned16(norm_weight) || !aligned16(weight))
-    return fail(HEXKV_EUNSUPPORTED, "%s: rows must be 16-byte aligned and a multiple of 16 bytes", what);
   const LinearArgs a{NormArgs{h, y, norm_weight, h_out, nullptr, h_stride, y_stride, h_out_stride, hidden, eps},
-                     weight, out, n};
+                     weight, out, n, RopeArgs{}};
+  const int bad = check_linear(a.norm, weight, rows, es, what);
+  if (bad != HEXKV_OK) return bad;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  switch (dtype) {
-    case HEXKV_BF16: dispatch_linear<__bf16>(a, rows, glu != 0, s); break;
-    case HEXKV_F16: dispatch_linear<_Float16>(a, rows, glu != 0, s); break;
-    default: dispatch_linear<float>(a, rows, glu != 0, s); break;
-  }
+  if (glu) dispatch_linear<kLinearGlu>(a, rows, dtype, s);
+  else dispatch_linear<kLinearPlain>(a, rows, dtype, s);
+  return check_launch(what);
+}
+
+extern "C" int hexkv_norm_rope_linear(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
+                                      int64_t h_out_stride, const void *norm_weight, float eps, const void *weight,
+                                      const float *inv_freq_dev, const int32_t *positions_dev, int offset, void *q,
+                                      void *kv, int rows, int seqlen, int hidden, int q_heads, int kv_heads,
+                                      int head_dim, int dtype, hexkv_stream_t stream) {
+  using namespace hexkv;
+  clear_error();
+  const char *what = "hexkv_norm_rope_linear";
+  int es = 0;
+  const int rc = dtype_size(dtype, what, &es);
+  if (rc != HEXKV_OK) return rc;
+  if (rows < 0 || hidden < 1 || q_heads < 1 || kv_heads < 1 || head_dim < 2 || head_dim % 2 || seqlen < 1 || rows % seqlen)
+    return fail(HEXKV_EINVAL, "%s: bad sizes", what);
+  const int64_t units = (static_cast<int64_t>(q_heads) + 2 * static_cast<int64_t>(kv_heads)) * (head_dim / 2);
+  if (units > 1 << 22) return fail(HEXKV_ERANGE, "%s: rows of more than 2^23 elements", what);
+  if (offset < 0 || (!positions_dev && offset > INT32_MAX - seqlen))
+    return fail(HEXKV_ERANGE, "%s: position offset %d", what, offset);
+  if (rows == 0) return HEXKV_OK;
+  if (!h || !weight || !inv_freq_dev || !q || !kv) return fail(HEXKV_EINVAL, "%s: null tensor", what);
+  const LinearArgs a{NormArgs{h, y, norm_weight, h_out, nullptr, h_stride, y_stride, h_out_stride, hidden, eps},
+                     weight, nullptr, static_cast<int32_t>(units),
+                     RopeArgs{nullptr, q, kv, inv_freq_dev, positions_dev, 0, q_heads, kv_heads, head_dim, seqlen, offset}};
+  const int bad = check_linear(a.norm, weight, rows, es, what);
+  if (bad != HEXKV_OK) return bad;
+  dispatch_linear<kLinearRope>(a, rows, dtype, static_cast<hipStream_t>(stream));
   return check_launch(what);
 }
 

@@ -146,14 +146,19 @@ class LlamaHost:
         h = F.embedding(input_ids, self.embed)
         y = None  # the block output still to be added to h
         for i, layer in enumerate(self.layers):
-            qkv, h = self._norm_linear(h, y, layer["ln1"], layer["wqkv"])
             if inference_params.fused_ft_kernel and offset > 0:
                 # FT decode (mha.py:553-571): rotary, append and attention in one call
+                qkv, h = self._norm_linear(h, y, layer["ln1"], layer["wqkv"])
                 q = qkv[..., :heads * d].view(batch, seqlen, heads, d)
                 kv = qkv[..., heads * d:].view(batch, seqlen, 2, kv_heads, d)
                 context = _apply_rotary_single_query_attention(q, inference_params, i, d, s.rope_theta, kv=kv)
             else:
-                q, kv = ops.rope_split(qkv, heads, kv_heads, d, self.inv_freq, offset, positions)
+                if ops.linear_fits(h, layer["ln1"], layer["wqkv"]):
+                    q, kv, h = ops.norm_rope_linear(h, y, layer["ln1"], s.rms_norm_eps, layer["wqkv"], heads, kv_heads, d,
+                                                    self.inv_freq, offset, positions)
+                else:
+                    qkv, h = self._norm_linear(h, y, layer["ln1"], layer["wqkv"])
+                    q, kv = ops.rope_split(qkv, heads, kv_heads, d, self.inv_freq, offset, positions)
                 if fused_append and offset > 0 and seqlen == 1 and i in inference_params.key_value_memory_dict:
                     context = update_and_attend(q, kv, inference_params, i, self.scale)
                 else:

@@ -743,17 +743,15 @@ def linear_fits(x: torch.Tensor, *weights: torch.Tensor) -> bool:
             and all(w.is_contiguous() and w.data_ptr() % 16 == 0 and w.dtype == x.dtype for w in weights))
 
 
-def norm_linear(h: torch.Tensor, y: Optional[torch.Tensor], norm_weight: Optional[torch.Tensor], eps: float,
-                weight: torch.Tensor, glu: bool = False, keep_sum: bool = True):
-    """``(out, sum)`` of up to 2 tokens in one launch: ``sum = h + y`` (``h``
-    itself without ``y``, not formed without ``keep_sum``), ``out =
-    rms_norm(sum) * norm_weight @ weight.T`` (``norm_weight`` None: ``h @
-    weight.T``), with ``glu`` ``silu(gate) * up`` of ``weight``'s two halves."""
+def _linear_inputs(h, y, norm_weight, weight, keep_sum):
+    """Checked inputs of the few-token products: the library's leading
+    arguments (h, y and where their sum goes, each with its row stride, the
+    norm's weight) and the sum's tensor (``h`` when none is formed)."""
     _require_device(h, weight)
     hidden = h.shape[-1]
     if h.dtype not in _DTYPES or weight.dtype != h.dtype or weight.device != h.device:
         raise ValueError("h and weight must share one of float16, bfloat16, float32 and a device")
-    if weight.dim() != 2 or weight.shape[1] != hidden or not weight.is_contiguous() or (glu and weight.shape[0] % 2):
+    if weight.dim() != 2 or weight.shape[1] != hidden or not weight.is_contiguous():
         raise ValueError(f"weight must be contiguous [n, {hidden}], got {tuple(weight.shape)}")
     norm_ptr = y_ptr = kept = None
     y_stride = 0
@@ -770,13 +768,56 @@ def norm_linear(h: torch.Tensor, y: Optional[torch.Tensor], norm_weight: Optiona
         if keep_sum:
             total = h.new_empty(h.shape)
             kept = total.data_ptr()
-    n = weight.shape[0] // 2 if glu else weight.shape[0]
+    return (h.data_ptr(), _row_stride(h, "h"), y_ptr, y_stride, kept, hidden, norm_ptr), total
+
+
+def norm_linear(h: torch.Tensor, y: Optional[torch.Tensor], norm_weight: Optional[torch.Tensor], eps: float,
+                weight: torch.Tensor, glu: bool = False, keep_sum: bool = True):
+    """``(out, sum)`` of up to 2 tokens in one launch: ``sum = h + y`` (``h``
+    itself without ``y``, not formed without ``keep_sum``), ``out =
+    rms_norm(sum) * norm_weight @ weight.T`` (``norm_weight`` None: ``h @
+    weight.T``), with ``glu`` ``silu(gate) * up`` of ``weight``'s two halves."""
+    inputs, total = _linear_inputs(h, y, norm_weight, weight, keep_sum)
+    hidden, n = h.shape[-1], weight.shape[0]
+    if glu:
+        if n % 2:
+            raise ValueError(f"weight holds {n} rows, not two halves")
+        n //= 2
     out = h.new_empty((*h.shape[:-1], n))
-    rc = _lib.load().hexkv_norm_linear(h.data_ptr(), _row_stride(h, "h"), y_ptr, y_stride, kept, hidden, norm_ptr, eps,
-                                       weight.data_ptr(), out.data_ptr(), h.numel() // hidden if hidden else 0, hidden,
-                                       n, 1 if glu else 0, _DTYPES[h.dtype], _stream(h))
+    rc = _lib.load().hexkv_norm_linear(*inputs, eps, weight.data_ptr(), out.data_ptr(),
+                                       h.numel() // hidden if hidden else 0, hidden, n, 1 if glu else 0,
+                                       _DTYPES[h.dtype], _stream(h))
     _lib.check(rc, "hexkv_norm_linear")
     return out, total
+
+
+def norm_rope_linear(h: torch.Tensor, y: Optional[torch.Tensor], norm_weight: torch.Tensor, eps: float,
+                     weight: torch.Tensor, q_heads: int, kv_heads: int, head_dim: int, inv_freq: torch.Tensor,
+                     offset: int = 0, positions: Optional[torch.Tensor] = None):
+    """``(q, kv, sum)`` of up to 2 tokens ``h [B, S, hidden]``: ``norm_linear``
+    with the q, k and v heads' rows of ``weight``, then ``rope_split``, in one
+    launch and rounded once."""
+    inputs, total = _linear_inputs(h, y, norm_weight, weight, True)
+    if h.dim() != 3 or weight.shape[0] != (q_heads + 2 * kv_heads) * head_dim:
+        raise ValueError(f"h must be [B, S, hidden] and weight [{(q_heads + 2 * kv_heads) * head_dim}, hidden]")
+    _require_device(inv_freq)
+    if inv_freq.dtype != torch.float32 or inv_freq.shape != (head_dim // 2,) or not inv_freq.is_contiguous() \
+            or inv_freq.device != h.device:
+        raise ValueError("inv_freq must be contiguous float32 [head_dim / 2] on h's device")
+    batch, seqlen, hidden = h.shape
+    pos_ptr = None
+    if positions is not None:
+        _require_device(positions)
+        if positions.dtype != torch.int32 or positions.numel() < batch or not positions.is_contiguous():
+            raise ValueError("positions must be a contiguous int32 device tensor with one entry per sequence")
+        pos_ptr = positions.data_ptr()
+    q = h.new_empty((batch, seqlen, q_heads, head_dim))
+    kv = h.new_empty((batch, seqlen, 2, kv_heads, head_dim))
+    rc = _lib.load().hexkv_norm_rope_linear(*inputs, eps, weight.data_ptr(), inv_freq.data_ptr(), pos_ptr, int(offset),
+                                            q.data_ptr(), kv.data_ptr(), batch * seqlen, max(seqlen, 1), hidden,
+                                            q_heads, kv_heads, head_dim, _DTYPES[h.dtype], _stream(h))
+    _lib.check(rc, "hexkv_norm_rope_linear")
+    return q, kv, total
 
 
 def _row_stride(t: torch.Tensor, name: str) -> int:

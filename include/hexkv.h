@@ -624,6 +624,14 @@ int hexkv_norm_linear(const void *h, int64_t h_stride, const void *y, int64_t y_
                       int64_t h_out_stride, const void *norm_weight, float eps, const void *weight,
                       void *out, int rows, int hidden, int n, int glu, int dtype, hexkv_stream_t stream);
 
+/* hexkv_norm_linear over the q, k and v heads' rows of W and hexkv_rope_split
+ * of its product, in one launch and rounded once. */
+int hexkv_norm_rope_linear(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
+                           int64_t h_out_stride, const void *norm_weight, float eps, const void *weight,
+                           const float *inv_freq_dev, const int32_t *positions_dev, int offset, void *q,
+                           void *kv, int rows, int seqlen, int hidden, int q_heads, int kv_heads,
+                           int head_dim, int dtype, hexkv_stream_t stream);
+
 /* Rows [q heads | k heads | v heads] of head_dim elements (qkv_stride apart)
  * into q [rows][q_heads][head_dim] and kv [rows][2][kv_heads][head_dim], q
  * and k rotated (GPT-NeoX halves) by position * inv_freq_dev[j].  Row r is

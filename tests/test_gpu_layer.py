@@ -112,6 +112,38 @@ def test_norm_linear(dtype, rows, hidden, n):
     _within(got, silu * u, bound + TINY)
 
 
+@pytest.mark.parametrize("dtype", DTYPES)
+@pytest.mark.parametrize("batch,seqlen,ragged", [(1, 1, False), (1, 2, False), (2, 1, False), (2, 1, True)])
+@pytest.mark.parametrize("hidden,heads,kv_heads,dim", [(64, 4, 4, 16), (2048, 32, 4, 64), (520, 8, 1, 128), (16, 3, 1, 6),
+                                                       (1024, 48, 8, 64)])
+def test_norm_rope_linear(dtype, batch, seqlen, ragged, hidden, heads, kv_heads, dim):
+    """Against the product of the same normalised tokens in 64 bits, turned
+    by the fp32 angle: the product's error turns with it."""
+    torch.manual_seed(hidden + batch)
+    offset = 0 if ragged else 4091
+    h, y = (torch.randn(batch, seqlen, hidden, device="cuda").to(dtype) for _ in range(2))
+    norm = torch.randn(hidden, device="cuda").to(dtype)
+    w = (torch.randn((heads + 2 * kv_heads) * dim, hidden, device="cuda") * hidden ** -0.5).to(dtype)
+    inv = 1.0 / (10000.0 ** (torch.arange(0, dim, 2, device="cuda", dtype=torch.float32) / dim))
+    at = torch.tensor([8191, 17], dtype=torch.int32, device="cuda") if ragged else None
+    total = h.clone()
+    x = ops.add_rms_norm(total, y, norm, 1e-5)
+    q, kv, kept = ops.norm_rope_linear(h, y, norm, 1e-5, w, heads, kv_heads, dim, inv, offset, at)
+    assert torch.equal(kept, total)
+    full = (x.double() @ w.double().T).view(batch, seqlen, -1, dim)
+    flip = 2 * UNIT[dtype] * (x.double().abs().amax() * w.double().abs().amax())
+    err = ((hidden + 63) // 64 + 8) * 2.0 ** -24 * (x.double().abs() @ w.double().abs().T).view(full.shape) + 8 * flip
+    pos = at.float()[:, None] if ragged else (offset + torch.arange(seqlen, device="cuda").float())[None].expand(batch, -1)
+    angle = (pos[..., None] * inv).double()[:, :, None]
+    a, b = full[..., :dim // 2], full[..., dim // 2:]
+    want = torch.cat((a * angle.cos() - b * angle.sin(), b * angle.cos() + a * angle.sin()), -1)
+    want[:, :, heads + kv_heads:] = full[:, :, heads + kv_heads:]
+    got = torch.cat((q, kv.flatten(2, 3)), 2)
+    size = (a.abs() + b.abs()).repeat(1, 1, 1, 2)
+    both = (err[..., :dim // 2] + err[..., dim // 2:]).repeat(1, 1, 1, 2)
+    _within(got, want, 1.01 * UNIT[dtype] * want.abs() + both + FP32 * size + TINY)
+
+
 def test_norm_linear_fits_and_refuses():
     x, w = torch.zeros(2, 1, 64, device="cuda").half(), torch.zeros(16, 64, device="cuda").half()
     assert ops.linear_fits(x, w)
