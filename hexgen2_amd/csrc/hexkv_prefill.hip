@@ -7,15 +7,21 @@
 // for the matrix cores, which bound this kernel (a softmax step per score on
 // the VALU beside them).
 //
+// Measured on MI355X against the decode kernels row by row: Llama-3-8B's
+// 8192-token layer 760-810 us and 16.9 ms, 700 TFLOP/s of the products
+// without the lo halves (1.05 PFLOP/s with them; a library product reaches
+// 1.2), matrix cores 53% and VALU 46% busy, LDS 26%; a Llama-2-7B chunk of
+// 2 x 611 over 512 keys 55 and 1165 us.
+//
 // Work split: a workgroup (4 waves) takes ROWS of the q_len * group query
 // rows that share one (sequence, KV head) pair, in (position, query head)
 // order, so a grouped query's heads share the staged keys and a tile spans
 // few positions (little work above the causal diagonal).  Consecutive
 // workgroups are different pairs: with the round-robin dispatch a pair's
 // tiles meet its K and V in one XCD's L2.  Tiles run from the longest rows
-// down.  When the tiles alone leave CUs idle (a short chunk over a long
-// past), the keys are cut into partitions merged by combine_kernel as for
-// decode rows.
+// down.  When the tiles alone leave CUs idle and the rows are few for their
+// keys (a short chunk over a long past), the keys are cut into partitions
+// merged by combine_kernel as for decode rows (tile_partition).
 //
 // One wave, 32 query rows (one per lane and half):
 //   S^T = K Q^T   v_mfma_f32_32x32x16, K (A) from LDS, Q (B) in registers:
