@@ -347,13 +347,18 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
   const bool bad = holds && lim > p0 && !(check == 0.f);
   if (holds && !bad) {
     if (nparts <= 1) {
-      const float inv = len > 0 ? 1.f / l : 0.f;
+      // A row without keys is zero, not its sum times zero: beside rows that
+      // attend an infinity its sum of 0 * V is a NaN.
+      const float inv = 1.f / l;
       T *out = static_cast<T *>(a.out) + b * a.o_bs + t * a.o_rs + static_cast<int64_t>(qh) * D + 4 * h;
 #pragma unroll
       for (int d = 0; d < ND; ++d)
 #pragma unroll
-        for (int i = 0; i < 4; ++i)
-          store4(out + d * 32 + i * 8, f32x4{acc[d][4 * i], acc[d][4 * i + 1], acc[d][4 * i + 2], acc[d][4 * i + 3]} * inv);
+        for (int i = 0; i < 4; ++i) {
+          f32x4 o = f32x4{acc[d][4 * i], acc[d][4 * i + 1], acc[d][4 * i + 2], acc[d][4 * i + 3]} * inv;
+          if (len <= 0) o = f32x4{};
+          store4(out + d * 32 + i * 8, o);
+        }
     } else {
       const int64_t slot = ((static_cast<int64_t>(b) * a.q_len + t) * a.q_heads + qh) * a.max_parts + part;
       float *o = a.ws_o + slot * D + 4 * h;

@@ -115,6 +115,22 @@ def test_non_finite_values_stay_in_their_rows(device, dtype, hq, hkv, d, partiti
         assert torch.equal(out[0, :, :hq // hkv], clean[0, :, :hq // hkv])  # the other KV head
 
 
+@pytest.mark.parametrize("dtype,hq,hkv,d", [(torch.float16, 4, 2, 64), (torch.bfloat16, 8, 2, 128)])
+@pytest.mark.parametrize("partition", [0, 64])
+@pytest.mark.parametrize("value", [float("inf"), float("nan")])
+def test_rows_without_keys_are_zero_beside_non_finite_values(device, dtype, hq, hkv, d, partition, value):
+    """A row that attends nothing is zero whatever the rows of its tile meet."""
+    q_len, n = 37, 20
+    q, cache = make(2, 80, hq, hkv, d, dtype, device, q_len)
+    cache[:, 0, 1, :, 3] = value
+    seqlens = torch.tensor([n, 80], dtype=torch.int32, device=device)
+    out = ops.decode_attention(q, cache, max_seqlen=80, seqlens=seqlens, causal=True, partition=partition)
+    assert torch.equal(out[0, :q_len - n], torch.zeros_like(out[0, :q_len - n]))
+    assert not bool(torch.isfinite(out[0, q_len - n:, :, 3]).any())
+    rest = [i for i in range(d) if i != 3]
+    assert bool(torch.isfinite(out[..., rest]).all())
+
+
 def test_lowest_scores_and_large_scales(device):
     """Scores at the type's lowest and highest values (softmax one-hot)."""
     q, cache = make(1, 90, 2, 1, 64, torch.bfloat16, device, 70)
