@@ -344,7 +344,11 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
   for (int d = 0; d < ND; ++d)
 #pragma unroll
     for (int i = 0; i < 16; ++i) check = fmaf(acc[d][i], 0.f, check);
-  const bool bad = holds && lim > p0 && !(check == 0.f);
+  // Decided for the row, over both lanes that hold its outputs, before either
+  // stores: `out` may be `q`, and exact_row reads the row's query again.
+  uint64_t redo = __ballot(holds && lim > p0 && !(check == 0.f));
+  redo = (redo | redo >> 32) & 0xffffffffu;
+  const bool bad = redo >> c & 1;
   if (holds && !bad) {
     if (nparts <= 1) {
       // A row without keys is zero, not its sum times zero: beside rows that
@@ -371,8 +375,6 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
       if (h == 0) *reinterpret_cast<float2 *>(a.ws_ml + slot * 2) = float2{m, l};
     }
   }
-  uint64_t redo = __ballot(bad);
-  redo = (redo | redo >> 32) & 0xffffffffu;
   while (redo) {
     const int r = __builtin_ctzll(redo);
     redo &= redo - 1;

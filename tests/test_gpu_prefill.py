@@ -131,6 +131,22 @@ def test_rows_without_keys_are_zero_beside_non_finite_values(device, dtype, hq, 
     assert bool(torch.isfinite(out[..., rest]).all())
 
 
+@pytest.mark.parametrize("dtype,hq,hkv,d", [(torch.float16, 4, 2, 64), (torch.bfloat16, 8, 2, 128)])
+@pytest.mark.parametrize("partition", [0, 64])
+@pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan"))])
+def test_out_may_be_q(device, dtype, hq, hkv, d, partition, where, value):
+    """In place, rows recomputed for a non-finite value read their own query:
+    the same results as into another tensor."""
+    q_len, n = 150, 170
+    q, cache = make(1, n, hq, hkv, d, dtype, device, q_len, seed=3)
+    cache[0, 95, "kv".index(where), 1, 3] = value
+    args = dict(max_seqlen=n, seqlen_bias=n, causal=True, partition=partition)
+    want = ops.decode_attention(q, cache, **args)
+    got = ops.decode_attention(q, cache, out=q, **args)
+    assert torch.equal(torch.isnan(got), torch.isnan(want))
+    assert torch.equal(got.nan_to_num(), want.nan_to_num())
+
+
 def test_lowest_scores_and_large_scales(device):
     """Scores at the type's lowest and highest values (softmax one-hot)."""
     q, cache = make(1, 90, 2, 1, 64, torch.bfloat16, device, 70)
