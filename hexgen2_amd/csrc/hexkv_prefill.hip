@@ -292,19 +292,22 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
 #pragma unroll
         for (int i = 0; i < 16; ++i) acc[d][i] *= f;
     }
+    // The tile's sum first: a probability alone may be below half a spacing of l.
+    float l0 = 0.f, l1 = 0.f;
     u32x4 hi[2 * NKB], lo[2 * NKB];
 #pragma unroll
     for (int kb = 0; kb < NKB; ++kb)
 #pragma unroll
       for (int i = 0; i < 16; i += 2) {
         const float e0 = tile_exp2(fmaf(s[kb][i], scale, -m)), e1 = tile_exp2(fmaf(s[kb][i + 1], scale, -m));
-        l += e0;
-        l += e1;
+        l0 += e0;
+        l1 += e1;
         unsigned int x, y;
         M::split(e0, e1, &x, &y);
         hi[2 * kb + i / 8][i % 8 / 2] = x;
         lo[2 * kb + i / 8][i % 8 / 2] = y;
       }
+    l += l0 + l1;
 #pragma unroll
     for (int ks = 0; ks < 2 * NKB; ++ks)
 #pragma unroll

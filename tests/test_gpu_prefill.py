@@ -156,6 +156,22 @@ def test_lowest_scores_and_large_scales(device):
     check(out, q, cache, [90], True)
 
 
+def test_sum_keeps_keys_far_below_the_largest(device):
+    """A probability of 1 and 2^20 - 1 of 2^-25.2, each below half a spacing of
+    the row's running sum: together 2.7% of it.  The call is large enough to
+    walk its keys unsplit.  Bound: the output's rounding and 2^-11 (2^20 / 64
+    fp32 additions of tile sums, half a spacing each, relative to the sum)."""
+    n, q_len, d = 1 << 20, 33024, 64
+    cache = torch.zeros(1, n, 2, 1, d, dtype=torch.bfloat16, device=device)
+    cache[:, 0, 0, 0, 0] = 17.5
+    cache[:, 0, 1] = 1
+    q = torch.zeros(1, q_len, 1, d, dtype=torch.bfloat16, device=device)
+    q[..., 0] = d ** 0.5  # scores are dimension 0 of the keys
+    out = f64(ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n)[:, ::997])
+    want = 1 / (1 + (n - 1) * np.exp(-17.5))
+    assert float(np.abs(out - want).max()) <= (2.0 ** -8 + 2.0 ** -11) * want
+
+
 def test_replay_matches_eager(device):
     q, cache = make(1, 2100, 8, 1, 128, torch.bfloat16, device, 9)
     out = torch.empty_like(q)
