@@ -28,13 +28,14 @@
 //                 lane (q, h) gets row q's scores of keys 8 i + 4 h + e.
 //   softmax       in the log2 domain per lane, one permlane32 exchange for
 //                 the maximum, the running maximum moved only when a score
-//                 exceeds it by 2^kSlack.
+//                 exceeds it by more than kSlack.
 //   O^T += V^T P^T the score layout is the B operand as it stands (the
 //                 contraction index of a 16-key step is key 4 h + e, then
 //                 8 + 4 h + e), V^T (A) comes from row-major LDS by
 //                 ds_read_b64_tr_b16 in the same order.  Every probability
 //                 enters as hi + lo 16-bit values (about 2^-17 relative for
-//                 bf16, 2^-21 for fp16), both products exact in fp32.
+//                 bf16; 2^-22 for fp16, or 2^-36 of the row's largest),
+//                 both products exact in fp32.
 // A lane's accumulators all belong to its own row, so rescaling and the
 // final division need no exchange.
 //
@@ -55,7 +56,6 @@ namespace hexkv {
 
 constexpr int kTileThreads = 256;
 constexpr int kTileWaves = kTileThreads / 64;
-constexpr float kSlack = 8.f;       // log2 units
 constexpr float kLowest = -1e30f;   // finite "minus infinity" of the running maximum
 
 typedef short h4 __attribute__((ext_vector_type(4)));
@@ -65,6 +65,10 @@ typedef __attribute__((address_space(3))) h4 lds_h4;
 
 __device__ __forceinline__ float tile_exp2(float x) { return __builtin_amdgcn_exp2f(x); }
 
+// Two 16-bit values per probability, and the scale they are held at: with
+// the running maximum M at the last move, a score s enters as
+// 2^(s - M + kShift), up to 2^(kShift + kSlack) before the maximum moves (all
+// in log2 units).  The scale cancels in the division by the row's sum.
 template <typename T>
 struct Mma32;
 
@@ -72,6 +76,9 @@ template <>
 struct Mma32<__bf16> {
   typedef __bf16 v8 __attribute__((ext_vector_type(8)));
   typedef __bf16 v2 __attribute__((ext_vector_type(2)));
+  // bf16 has fp32's exponents: no probability is too small, and a larger
+  // scale would only bring P V closer to fp32's range.
+  static constexpr float kShift = 0.f, kSlack = 8.f;
   __device__ __forceinline__ static f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_bf16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
   }
@@ -89,6 +96,14 @@ template <>
 struct Mma32<_Float16> {
   typedef _Float16 v8 __attribute__((ext_vector_type(8)));
   typedef _Float16 v2 __attribute__((ext_vector_type(2)));
+  // fp16 ends at 2^-24 (rounded: 2^-25), so at scale 1 a probability below
+  // 2^-25 of the largest was lost to the product though not to the sum: one
+  // high score over 65536 keys just below took the whole output.  At 2^11
+  // the loss is below 2^-36 a key (2^-20 over 65536 keys), and 2^(11 + 4)
+  // still lies below fp16's 65504.  A smaller slack moves the maximum more
+  // often: a Llama-2-7B chunk of 2 x 611 over 512 keys takes 54.8 us with a
+  // slack of 8 (scale 2^7), 55.2 with 4 and 56.0 with 2 (2^13).
+  static constexpr float kShift = 11.f, kSlack = 4.f;
   __device__ __forceinline__ static f32x16 mma(u32x4 a, u32x4 b, f32x16 c) {
     return __builtin_amdgcn_mfma_f32_32x32x16_f16(__builtin_bit_cast(v8, a), __builtin_bit_cast(v8, b), c, 0, 0, 0);
   }
@@ -137,7 +152,7 @@ __device__ __forceinline__ void exact_row(const TileArgs &a, int b, int t, int q
                  *reinterpret_cast<const u32x4 *>(kseq + static_cast<int64_t>(pos) * a.c_ps + c), s);
     if (k0 + lane >= end) s = -INFINITY;
     const float mt = wave_max(s) * a.scale_log2;
-    if (mt > m + kSlack) {
+    if (mt > m + 8.f) {
       const float c = tile_exp2(m - mt);
       m = mt;
       l *= c;
@@ -227,7 +242,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
   const uint32_t row_bytes = static_cast<uint32_t>(a.c_ps * sizeof(T));
   const float scale = a.scale_log2;
 
-  float m = kLowest, l = 0.f;
+  float m = kLowest, l = 0.f;  // m: the running maximum less kShift
   f32x16 acc[ND];
 #pragma unroll
   for (int d = 0; d < ND; ++d) acc[d] = f32x16{};
@@ -281,9 +296,9 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
 #pragma unroll
       for (int i = 0; i < 16; ++i) mt = fmaxf(mt, s[kb][i]);
     mt = other_half_max(mt) * scale;
-    const bool up = mt > m + kSlack;
+    const bool up = mt > m + (M::kShift + M::kSlack);
     if (__any(up)) {
-      const float mnew = up ? mt : m;
+      const float mnew = up ? mt - M::kShift : m;
       const float f = tile_exp2(m - mnew);
       m = mnew;
       l *= f;

@@ -172,6 +172,30 @@ def test_sum_keeps_keys_far_below_the_largest(device):
     assert float(np.abs(out - want).max()) <= (2.0 ** -8 + 2.0 ** -11) * want
 
 
+@pytest.mark.parametrize("dtype,high", [(torch.float16, 17.46875), (torch.float16, 22.0), (torch.bfloat16, 17.5)])
+@pytest.mark.parametrize("first", [True, False])
+def test_many_keys_far_below_one(device, dtype, high, first):
+    """One score exp(17) above 65535 others, whose values still make up the
+    output (the high one's are zero): no probability may be lost.  The call is
+    large enough to walk its keys unsplit.  Bound: the output's rounding,
+    65536 / 16 fp32 additions (the sum has as many), and for fp16 2^-36 of the
+    largest probability per key, times values below 2."""
+    n, q_len, heads, d = 65536, 4224, 8, 64
+    g = torch.Generator(device=device).manual_seed(1)
+    cache = torch.zeros(1, n, 2, heads, d, dtype=dtype, device=device)
+    cache[:, :, 1] = (1 + torch.rand(1, n, heads, d, generator=g, device=device)).to(dtype)
+    at = 0 if first else n - 1
+    cache[:, at, 0, :, 0] = high
+    cache[:, at, 1] = 0
+    q = torch.zeros(1, q_len, heads, d, dtype=dtype, device=device)
+    q[..., 0] = d ** 0.5  # scores are dimension 0 of the keys
+    out = f64(ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n)[:, ::97])
+    want = oracle.attend(f64(q[:, :1]), f64(cache), [n])
+    u = {torch.float16: 2.0 ** -11, torch.bfloat16: 2.0 ** -8}[dtype]
+    bound = (u + 2 * n / 16 * 2.0 ** -24) * want + 2.0 ** -25 + n * 2.0 ** -36 * 2
+    assert (np.abs(out - want) <= bound).all(), float((np.abs(out - want) / bound).max())
+
+
 def test_replay_matches_eager(device):
     q, cache = make(1, 2100, 8, 1, 128, torch.bfloat16, device, 9)
     out = torch.empty_like(q)
