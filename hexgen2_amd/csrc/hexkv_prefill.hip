@@ -129,7 +129,8 @@ __device__ __forceinline__ int keys_of(const TileArgs &a, int base, int t) {
 
 // Row (position t, query head qh) over keys [p0, end) by one wave, key by key
 // in fp32: lanes hold a key each for the scores, D / 64 outputs each for the
-// values.  Used for rows whose tile result is not finite.
+// values.  Used for rows whose tile result is not finite, values past
+// fp32's range at the tile's scale among them, so no probability exceeds 1.
 template <typename T, int D>
 __device__ __forceinline__ void exact_row(const TileArgs &a, int b, int t, int qh, int p0, int end, int nparts, int part) {
   using E = Elem<T>;
@@ -152,7 +153,7 @@ __device__ __forceinline__ void exact_row(const TileArgs &a, int b, int t, int q
                  *reinterpret_cast<const u32x4 *>(kseq + static_cast<int64_t>(pos) * a.c_ps + c), s);
     if (k0 + lane >= end) s = -INFINITY;
     const float mt = wave_max(s) * a.scale_log2;
-    if (mt > m + 8.f) {
+    if (mt > m) {
       const float c = tile_exp2(m - mt);
       m = mt;
       l *= c;

@@ -196,6 +196,22 @@ def test_many_keys_far_below_one(device, dtype, high, first):
     assert (np.abs(out - want) <= bound).all(), float((np.abs(out - want) / bound).max())
 
 
+@pytest.mark.parametrize("partition", [256, 128])
+def test_values_near_the_largest_number(device, partition):
+    """Rows whose maximum rises by less than the tile kernel's slack over
+    values near bf16's largest: no sum may pass fp32's range, as none does in
+    the per-row kernel."""
+    q_len, n, d = 40, 200, 64
+    cache = torch.zeros(1, n, 2, 1, d, dtype=torch.bfloat16, device=device)
+    cache[:, 130, 0, 0, 0] = 5.0  # 2^7.2 times the weight of any other key
+    cache[:, 130, 1] = 1e37
+    q = torch.zeros(1, q_len, 2, d, dtype=torch.bfloat16, device=device)
+    q[..., 0] = d ** 0.5
+    out = ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n, partition=partition)
+    want = oracle.attend(f64(q), f64(cache), [n])
+    assert float(np.abs(f64(out) / want - 1).max()) <= 2.0 ** -8 + 2.0 ** -16
+
+
 def test_replay_matches_eager(device):
     q, cache = make(1, 2100, 8, 1, 128, torch.bfloat16, device, 9)
     out = torch.empty_like(q)
