@@ -227,9 +227,11 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
   const int t = row / a.group, qh = hk * a.group + row - t * a.group;
   const int len = keys_of(a, base, t);
   const int lim = min(len, p0 + a.part);  // keys [p0, lim) are this lane's
-  const int w_end = wrow0 < total
-                        ? min(keys_of(a, base, (min(wrow0 + 32, total) - 1) / a.group), p0 + a.part) : p0;
-  const int w_full = min(keys_of(a, base, min(wrow0, total - 1) / a.group), p0 + a.part);  // below it no row masks
+  // Keys the wave walks, and those below which none of its rows masks; a wave
+  // without rows (the last tile of a pair) only stages.
+  const bool idle = wrow0 >= total;
+  const int w_end = idle ? p0 : min(keys_of(a, base, (min(wrow0 + 32, total) - 1) / a.group), p0 + a.part);
+  const int w_full = idle ? p0 : min(keys_of(a, base, wrow0 / a.group), p0 + a.part);
 
   u32x4 qf[NJ];
   {
@@ -354,7 +356,7 @@ __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const Tile
     }
   }
 
-  if (wrow0 >= total) return;
+  if (idle) return;
   l = xor_step<32>(l, AddOp{});
   const int nparts = len > 0 ? (len + a.part - 1) / a.part : 0;
   const bool holds = live && (part == 0 || lim > p0);  // this lane's row has something to write
