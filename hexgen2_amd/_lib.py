@@ -12,6 +12,7 @@ LIBRARY = Path(__file__).resolve().parent / "libhexkv.so"
 
 HEXKV_F16, HEXKV_BF16, HEXKV_F32 = 0, 1, 2
 KERNELS = {"auto": 0, "valu": 1, "mfma": 2, "rows": 3}
+KERNEL_NAMES = {**{v: k for k, v in KERNELS.items()}, 4: "tiles"}  # what hexkv_attend_kernel answers
 HEXKV_OK = 0
 HEXKV_EINVAL, HEXKV_ERANGE, HEXKV_EHIP, HEXKV_EUNSUPPORTED, HEXKV_EWORKSPACE = -1, -2, -3, -4, -5
 MAX_LAYERS_PER_LAUNCH = 96

@@ -2215,6 +2215,7 @@ extern "C" int hexkv_attend_kernel(const hexkv_attend_params *p) {
   if (p->kernel < HEXKV_KERNEL_AUTO || p->kernel > HEXKV_KERNEL_ROWS)
     return fail(HEXKV_EINVAL, "hexkv_attend_kernel: unknown kernel %d", p->kernel);
   if (p->kernel == HEXKV_KERNEL_ROWS) return HEXKV_KERNEL_ROWS;
+  if (use_tiles(p)) return HEXKV_KERNEL_TILES;
   return use_mfma(p, kernel_group(p->q_heads / p->kv_heads)) ? HEXKV_KERNEL_MFMA : HEXKV_KERNEL_VALU;
 }
 

@@ -47,19 +47,23 @@ enum hexkv_dtype {
   HEXKV_F32 = 2   /* torch.float32  */
 };
 
-/* Attention kernels.  AUTO picks MFMA for 16-bit data with head_dim 64 or
- * 128 and 8+ query heads per KV head, VALU otherwise; a work list is planned
- * and launched with hexkv_attend_plan_kernel's choice, which is ROWS for
- * AUTO on large calls. */
+/* Attention kernels.  AUTO picks TILES for 16-bit data with head_dim 64 or
+ * 128 and q_len > 1, else MFMA for such data with 8+ query heads per KV head,
+ * VALU otherwise; a work list is planned and launched with
+ * hexkv_attend_plan_kernel's choice, which is ROWS for AUTO on large calls. */
 enum hexkv_kernel {
   HEXKV_KERNEL_AUTO = 0,
   HEXKV_KERNEL_VALU = 1, /* packed dot products on the vector ALUs     */
   HEXKV_KERNEL_MFMA = 2, /* scores and P.V on the matrix cores           */
-  HEXKV_KERNEL_ROWS = 3  /* work lists planned for the XCDs only: each item
+  HEXKV_KERNEL_ROWS = 3, /* work lists planned for the XCDs only: each item
                             covers a block of adjacent KV heads (contiguous
                             bytes of every cache row); 16-bit, head_dim 128,
                             1, 2 or 4 query heads per KV head; see
                             hexkv_attend_plan_kernel */
+  HEXKV_KERNEL_TILES = 4 /* AUTO's kernel for several query rows per
+                            sequence (tiles of rows that share a KV head);
+                            an answer of hexkv_attend_kernel, refused as a
+                            request */
 };
 
 enum hexkv_status {
@@ -273,9 +277,8 @@ typedef struct hexkv_attend_params {
 #define HEXKV_ATTEND_COUNTER_BYTES (256u << 10)
 size_t hexkv_attend_workspace_bytes(const hexkv_attend_params *p);
 
-/* The kernel hexkv_attend runs for these parameters, HEXKV_KERNEL_VALU or
- * HEXKV_KERNEL_MFMA (HEXKV_KERNEL_AUTO resolved by head group, head_dim and
- * dtype), or a negative error code.  No counterpart in the reference: it
+/* The kernel hexkv_attend runs for these parameters (HEXKV_KERNEL_AUTO
+ * resolved as enum hexkv_kernel says), or a negative error code.  No counterpart in the reference: it
  * lets profiling and benchmarks name the kernel they measure. */
 int hexkv_attend_kernel(const hexkv_attend_params *p);
 

@@ -164,6 +164,20 @@ def test_attend_kernel_choice(hq, hkv, d, dtype, kernel, expect):
     assert ops.attend_kernel(q, cache, kernel) == expect
 
 
+@pytest.mark.parametrize("dtype,d,kernel,expect", [
+    (torch.float16, 128, "auto", "tiles"), (torch.bfloat16, 64, "auto", "tiles"),
+    (torch.float16, 128, "valu", "valu"), (torch.bfloat16, 64, "mfma", "mfma"),
+    (torch.float32, 128, "auto", "valu"), (torch.float16, 256, "auto", "valu")])
+def test_attend_kernel_choice_for_several_query_rows(dtype, d, kernel, expect):
+    """AUTO's kernel for q_len > 1 is named as the one that runs, and is no
+    kernel to ask for."""
+    q = torch.empty((2, 100, 8, d), dtype=dtype)
+    cache = torch.empty((2, 5000, 2, 8, d), dtype=dtype)
+    assert ops.attend_kernel(q, cache, kernel) == expect
+    with pytest.raises(ValueError):
+        ops.attend_kernel(q, cache, "tiles")
+
+
 def test_attend_kernel_rejects_bad_geometry():
     p = _lib.AttendParams()
     p.q_heads, p.kv_heads = 6, 4
