@@ -588,7 +588,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
 
   // One iteration covers U slots of one position per lane group.  `fetch`
   // issues its loads; TAIL clamps the positions past n_cache to the last
-  // cached one (finite data) and `consume` masks their scores.
+  // cached one and `consume` masks their scores and values.
   using Slots = u32x4[U][NV];
   auto fetch = [&](int i0, Slots &kr, Slots &vr, auto tail) {
     constexpr bool TAIL = decltype(tail)::value;
@@ -645,6 +645,13 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
       float vf[EPL];
 #pragma unroll
       for (int v = 0; v < NV; ++v) E::to_float(vr[u][v], vf + v * VEC);
+      if constexpr (TAIL) {
+        // a clamped position's value may be an infinity: zero times it is not zero
+        if (!(i0 + u * NG + gid < w.n_cache)) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) vf[e] = 0.f;
+        }
+      }
 #pragma unroll
       for (int g = 0; g < G; ++g) {
         const float pr = fast_exp2(fmaf(sc[u][g], scale, -m[g]));
@@ -809,7 +816,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_valu_kernel(const AttendAr
     lazy_rescale<G, EPL>(mt, m, l, acc);
     float vf[EPL];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) E::to_float(vn[v], vf + v * VEC);
+    for (int v = 0; v < NV; ++v) E::to_float(gid == 0 ? vn[v] : u32x4{}, vf + v * VEC);
 #pragma unroll
     for (int g = 0; g < G; ++g) {
       const float pr = fast_exp2(fmaf(sc[g], scale, -m[g]));
@@ -919,8 +926,8 @@ __global__ __launch_bounds__(kAttThreads) void attend_rows_kernel(const AttendAr
   }
 
   // Slot u of the iteration at i0 holds position i0 + u * PS + ps; TAIL
-  // clamps positions past n_cache to the last cached one (finite data) and
-  // `consume` masks their scores.
+  // clamps positions past n_cache to the last cached one and
+  // `consume` masks their scores and values.
   using Slots = u32x4[U][NV];
   auto fetch = [&](int i0, Slots &kr, Slots &vr, auto tail) {
     constexpr bool TAIL = decltype(tail)::value;
@@ -974,6 +981,13 @@ __global__ __launch_bounds__(kAttThreads) void attend_rows_kernel(const AttendAr
       float vf[EPL];
 #pragma unroll
       for (int v = 0; v < NV; ++v) E::to_float(vr[u][v], vf + v * VEC);
+      if constexpr (TAIL) {
+        // a clamped position's value may be an infinity: zero times it is not zero
+        if (!(i0 + u * PS + ps < w.n_cache)) {
+#pragma unroll
+          for (int e = 0; e < EPL; ++e) vf[e] = 0.f;
+        }
+      }
 #pragma unroll
       for (int g = 0; g < GQ; ++g) {
         const float pr = fast_exp2(fmaf(sc[u][g], scale, -m[g]));
@@ -1036,7 +1050,7 @@ __global__ __launch_bounds__(kAttThreads) void attend_rows_kernel(const AttendAr
     lazy_rescale<GQ, EPL>(mt, m, l, acc);
     float vf[EPL];
 #pragma unroll
-    for (int v = 0; v < NV; ++v) E::to_float(vn[v], vf + v * VEC);
+    for (int v = 0; v < NV; ++v) E::to_float(ps == 0 ? vn[v] : u32x4{}, vf + v * VEC);
 #pragma unroll
     for (int g = 0; g < GQ; ++g) {
       const float pr = fast_exp2(fmaf(sc[g], scale, -m[g]));
@@ -1192,8 +1206,10 @@ __global__ __launch_bounds__(kAttThreads, 3) void attend_mfma_kernel(const Atten
   // (MODE 0 full, 1 tail: positions past n_cache clamped to the last cached
   // one, 2: the new row from kv_new in every slot, written to the cache by
   // the writer); `consume` computes it (masking what MODE 1 and 2 do not
-  // attend).  Every staged V row holds finite data, so masked (zero)
-  // probabilities contribute exact zeros.
+  // attend).  A staged V row of a position not attended repeats one that is,
+  // so its zero probability adds an exact zero where the row's result is
+  // finite.  (An infinity in V gives NaN here: a probability's lo half may be
+  // zero.)
   auto fetch = [&](int i0, u32x4 (&kr)[NJ], u32x4 (&vr)[UV], auto mode) {
     constexpr int MODE = decltype(mode)::value;
     if constexpr (MODE == 2) {

@@ -517,3 +517,25 @@ def test_rows_with_hundreds_of_partitions(device, hq, hkv, d, dtype, kernel):
         err = (np.abs(f64(out)[live] - ref) / np.maximum(1.0, np.abs(ref))).max()
         assert err <= TOL[dtype], f"{'work list' if listed else 'grid'}: max-abs {err}"
         assert (out[2] == 0).all(), "empty row not zero"
+
+
+@pytest.mark.parametrize("kernel,hq,hkv,dtype", [("valu", 8, 2, torch.float16), ("valu", 2, 2, torch.float32),
+                                                 ("valu", 16, 2, torch.bfloat16), ("rows", 8, 2, torch.float16),
+                                                 ("rows", 2, 2, torch.bfloat16)])
+@pytest.mark.parametrize("new", [False, True])
+@pytest.mark.parametrize("n", [1, 17, 150, 300])
+def test_infinity_in_the_last_value(device, kernel, hq, hkv, dtype, new, n):
+    """The fp32 kernels: positions past a row's end repeat its last one with
+    probability zero, and an infinity there reaches the output as one, not as
+    zero times infinity."""
+    g = torch.Generator(device=device).manual_seed(n)
+    q = torch.randn((2, 1, hq, 128), generator=g, device=device).to(dtype)
+    cache = torch.randn((2, n + 20, 2, hkv, 128), generator=g, device=device).to(dtype)
+    kv = torch.randn((2, 2, hkv, 128), generator=g, device=device).to(dtype) if new else None
+    (kv[:, 1] if new else cache[:, n - 1, 1])[:, 1, 3] = float("inf")
+    lens = [n - 1 if new else n] * 2
+    out = ops.decode_attention(q, cache, max_seqlen=n, seqlens=torch.tensor(lens, dtype=torch.int32, device=device),
+                               kv_new=kv, kernel=kernel, lens=lens if kernel == "rows" else None)
+    assert bool((out[:, 0, hq // hkv:, 3] == float("inf")).all())
+    out[:, 0, hq // hkv:, 3] = 0
+    assert bool(torch.isfinite(out).all())
