@@ -1588,11 +1588,48 @@ static int choose_partition(const hexkv_attend_params *p) {
   return part;
 }
 
+static bool use_mfma(const hexkv_attend_params *p, int G);
+
+// Whether the per-row kernels lead for a call of several query rows: where
+// their workgroups (one per row, head group and 128 positions) run at once
+// and have little to read, or where a tile would hold four rows or fewer over
+// one partition.  The tile kernel's staging, barriers and 128-row tiles then
+// cost more than the keys it saves.  Lines from 4000 random calls (14
+// geometries of group 1-16, 1-64 sequences, 2-200 rows, up to 16000 keys):
+// by this rule 15 of them take over 1.1 times the per-row kernels' time (at
+// most 1.36), the tile kernel for all of them 1500 (at most 2.1), and the
+// geometric mean is within 1% of the faster kernel for each.  Tiles and
+// per-row kernel, us: TinyLlama, 16 rows over 100 keys 6.2 and 4.0, 64 over
+// 8000 21.6 and 55.9; Llama-2-7B 16 over 100 7.1 and 4.5, 64 over 1000 22 and
+// 62; Llama-2-70B TP-8 share 16 over 1000 11.2 and 7.5, 64 over 8000 19 and 53.
+constexpr int64_t kRowItems = 1280;
+constexpr int64_t kRowWork = INT64_C(24) << 20;  // elements of K its heads multiply
+constexpr int64_t kFewRows = 4;
+
+static int64_t row_work_per_key(const hexkv_attend_params *p) {
+  const int G = kernel_group(p->q_heads / p->kv_heads);
+  const int64_t heads = static_cast<int64_t>(p->batch) * p->q_len * p->q_heads;
+  return heads * p->head_dim * (use_mfma(p, G) ? 3 : 8);  // eighths: the MFMA kernel's cost less
+}
+
+static bool rows_lead(const hexkv_attend_params *p) {
+  const int group = p->q_heads / p->kv_heads;
+  const int64_t segments = static_cast<int64_t>(p->batch) * p->q_len * (p->q_heads / kernel_group(group));
+  const int64_t parts = (static_cast<int64_t>(p->max_seqlen) + 127) / 128;
+  if (segments * parts <= kRowItems && row_work_per_key(p) * p->max_seqlen <= 8 * kRowWork) return true;
+  const int64_t per = tile_rows(static_cast<int64_t>(p->q_len) * group);
+  const int64_t tiles = static_cast<int64_t>(p->batch) * p->kv_heads * ((static_cast<int64_t>(p->q_len) * group + per - 1) / per);
+  return parts <= 1 && segments <= kFewRows * tiles;
+}
+
 // Whether a call runs the query-tile kernel (hexkv_prefill.hip): several
-// query rows per sequence, AUTO, 16-bit data of head_dim 64 or 128.  An
-// explicit VALU or MFMA request keeps the per-row kernel it names.
+// query rows per sequence, AUTO, 16-bit data of head_dim 64 or 128, too many
+// rows and keys for the per-row kernels.  An explicit VALU or MFMA request
+// keeps the per-row kernel it names; an explicit partition keeps the tiles it
+// is meant for.
 static bool use_tiles(const hexkv_attend_params *p) {
-  return p->q_len > 1 && p->kernel == HEXKV_KERNEL_AUTO && tiles_support(p->dtype, p->head_dim);
+  return p->q_len > 1 && p->kernel == HEXKV_KERNEL_AUTO && tiles_support(p->dtype, p->head_dim) &&
+         (p->partition > 0 || !rows_lead(p));
 }
 
 // Partition size of a tile call: all keys in one partition unless splitting

@@ -374,11 +374,13 @@ def attend_workspace_bytes(q: torch.Tensor, cache: torch.Tensor, max_seqlen: int
     return int(_lib.load().hexkv_attend_workspace_bytes(ctypes.byref(p)))
 
 
-def attend_kernel(q: torch.Tensor, cache: torch.Tensor, kernel: str = "auto") -> str:
+def attend_kernel(q: torch.Tensor, cache: torch.Tensor, kernel: str = "auto",
+                  max_seqlen: Optional[int] = None, partition: int = 0) -> str:
     """Name of the kernel ("valu", "mfma" or, for several query rows per
-    sequence, "tiles") ``decode_attention`` runs for this geometry and
-    ``kernel`` choice."""
-    p = _attend_params(q, cache, q, None, 1, 1, None, False, None, 0, kernel)
+    sequence, "tiles") ``decode_attention`` runs for this geometry, ``kernel``
+    choice and ``max_seqlen`` (default: the cache's capacity)."""
+    longest = cache.shape[1] if max_seqlen is None else int(max_seqlen)
+    p = _attend_params(q, cache, q, None, longest, longest, None, False, None, partition, kernel)
     rc = int(_lib.load().hexkv_attend_kernel(ctypes.byref(p)))
     _lib.check(min(rc, 0), "hexkv_attend_kernel")
     return _lib.KERNEL_NAMES[rc]

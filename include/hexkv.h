@@ -48,8 +48,8 @@ enum hexkv_dtype {
 };
 
 /* Attention kernels.  AUTO picks TILES for 16-bit data with head_dim 64 or
- * 128 and q_len > 1, else MFMA for such data with 8+ query heads per KV head,
- * VALU otherwise; a work list is planned and launched with
+ * 128 and q_len > 1 unless the call is small (few rows or keys, by max_seqlen),
+ * else MFMA for such data with 8+ query heads per KV head, VALU otherwise; a work list is planned and launched with
  * hexkv_attend_plan_kernel's choice, which is ROWS for AUTO on large calls. */
 enum hexkv_kernel {
   HEXKV_KERNEL_AUTO = 0,

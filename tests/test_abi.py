@@ -178,6 +178,32 @@ def test_attend_kernel_choice_for_several_query_rows(dtype, d, kernel, expect):
         ops.attend_kernel(q, cache, "tiles")
 
 
+@pytest.mark.parametrize("batch,q_len,hq,hkv,d,longest,expect", [
+    (1, 40, 32, 32, 128, 128, "valu"),    # 1280 workgroups of one partition
+    (1, 41, 32, 32, 128, 128, "tiles"),
+    (1, 20, 32, 32, 128, 129, "valu"),    # two partitions each
+    (1, 20, 32, 32, 128, 257, "tiles"),
+    (1, 2, 32, 8, 128, 3072, "valu"),     # 24 Mi elements of K for the heads
+    (1, 2, 32, 8, 128, 3073, "tiles"),
+    (1, 2, 8, 1, 128, 32768, "mfma"),     # on the matrix cores 64 Mi
+    (1, 2, 8, 1, 128, 32769, "tiles"),
+    (32, 4, 32, 32, 128, 128, "valu"),    # four rows a tile over one partition
+    (32, 4, 32, 32, 128, 129, "tiles"),
+    (32, 5, 32, 32, 128, 128, "tiles")])
+def test_several_query_rows_take_the_kernel_that_leads(batch, q_len, hq, hkv, d, longest, expect):
+    """The lines between the per-row kernels and the query tiles; an explicit
+    partition takes the tiles on both sides."""
+    def name(longest, partition=0):
+        p = _lib.AttendParams(dtype=_lib.HEXKV_F16, batch=batch, q_len=q_len, q_heads=hq, kv_heads=hkv, head_dim=d,
+                              capacity=longest, max_seqlen=longest, softmax_scale=1.0, partition=partition)
+        return _lib.KERNEL_NAMES[_lib.load().hexkv_attend_kernel(ctypes.byref(p))]
+
+    assert name(longest) == expect and name(longest, 64) == "tiles"
+    # one line: every shorter call of a per-row length is a per-row call too
+    names = [name(n) for n in range(1, longest + 1, max(1, longest // 500))]
+    assert names == sorted(names, key=lambda k: k == "tiles")
+
+
 def test_attend_kernel_rejects_bad_geometry():
     p = _lib.AttendParams()
     p.q_heads, p.kv_heads = 6, 4

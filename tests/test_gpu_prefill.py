@@ -44,13 +44,16 @@ LENGTHS = [(2, 0), (6, 4090), (31, 0), (32, 1), (33, 31), (64, 0), (65, 63), (12
 
 @pytest.mark.parametrize("q_len,past", LENGTHS)
 @pytest.mark.parametrize("dtype,hq,hkv,d", GEOMETRIES)
-def test_tiles_match_the_oracle(device, dtype, hq, hkv, d, q_len, past):
+@pytest.mark.parametrize("partition", [0, 4096])
+def test_tiles_match_the_oracle(device, dtype, hq, hkv, d, q_len, past, partition):
+    """With a partition the tile kernel whatever the size, without one the
+    kernel that leads."""
     n = past + q_len
     q, cache = make(2, n + 3, hq, hkv, d, dtype, device, q_len)
-    out = ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n, causal=True)
+    out = ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n, causal=True, partition=partition)
     check(out, q, cache, [n, n], True)
     if q_len < 130:
-        out = ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n)
+        out = ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n, partition=partition)
         check(out, q, cache, [n, n], False)
 
 
@@ -82,7 +85,7 @@ def test_ragged_lengths_strides_and_partitions(device, dtype, hq, hkv, d, partit
 
 
 @pytest.mark.parametrize("dtype,hq,hkv,d", [(torch.float16, 4, 2, 64), (torch.bfloat16, 8, 2, 128)])
-@pytest.mark.parametrize("partition", [0, 64])
+@pytest.mark.parametrize("partition", [0, 64, 4096])
 @pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan")),
                                          ("k", float("inf")), ("q", float("nan"))])
 def test_non_finite_values_stay_in_their_rows(device, dtype, hq, hkv, d, partition, where, value):
@@ -100,8 +103,7 @@ def test_non_finite_values_stay_in_their_rows(device, dtype, hq, hkv, d, partiti
     ref = ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n, causal=True, partition=partition, kernel="valu")
     assert torch.equal(torch.isfinite(out), torch.isfinite(ref))
     if where == "v" and value == float("inf"):
-        # p * inf is inf for every attending row (the per-row kernel may give
-        # NaN where the infinity is the row's last key)
+        # p * inf is inf for every attending row
         assert bool((out[0, 75:, hq // hkv:, 3] == value).all())
     else:
         assert torch.equal(torch.isnan(out), torch.isnan(ref))
@@ -116,7 +118,7 @@ def test_non_finite_values_stay_in_their_rows(device, dtype, hq, hkv, d, partiti
 
 
 @pytest.mark.parametrize("dtype,hq,hkv,d", [(torch.float16, 4, 2, 64), (torch.bfloat16, 8, 2, 128)])
-@pytest.mark.parametrize("partition", [0, 64])
+@pytest.mark.parametrize("partition", [0, 64, 4096])
 @pytest.mark.parametrize("value", [float("inf"), float("nan")])
 def test_rows_without_keys_are_zero_beside_non_finite_values(device, dtype, hq, hkv, d, partition, value):
     """A row that attends nothing is zero whatever the rows of its tile meet."""
@@ -132,7 +134,7 @@ def test_rows_without_keys_are_zero_beside_non_finite_values(device, dtype, hq, 
 
 
 @pytest.mark.parametrize("dtype,hq,hkv,d", [(torch.float16, 4, 2, 64), (torch.bfloat16, 8, 2, 128)])
-@pytest.mark.parametrize("partition", [0, 64])
+@pytest.mark.parametrize("partition", [0, 64, 4096])
 @pytest.mark.parametrize("where,value", [("v", float("inf")), ("v", float("nan")), ("k", float("nan"))])
 def test_out_may_be_q(device, dtype, hq, hkv, d, partition, where, value):
     """In place, rows recomputed for a non-finite value read their own query:
@@ -147,12 +149,13 @@ def test_out_may_be_q(device, dtype, hq, hkv, d, partition, where, value):
     assert torch.equal(got.nan_to_num(), want.nan_to_num())
 
 
-def test_lowest_scores_and_large_scales(device):
+@pytest.mark.parametrize("partition", [0, 4096])
+def test_lowest_scores_and_large_scales(device, partition):
     """Scores at the type's lowest and highest values (softmax one-hot)."""
     q, cache = make(1, 90, 2, 1, 64, torch.bfloat16, device, 70)
     q *= 1e4
     cache[:, :, 0] *= 1e4
-    out = ops.decode_attention(q, cache, max_seqlen=90, seqlen_bias=90, causal=True)
+    out = ops.decode_attention(q, cache, max_seqlen=90, seqlen_bias=90, causal=True, partition=partition)
     check(out, q, cache, [90], True)
 
 
@@ -212,11 +215,13 @@ def test_values_near_the_largest_number(device, partition):
     assert float(np.abs(f64(out) / want - 1).max()) <= 2.0 ** -8 + 2.0 ** -16
 
 
-def test_replay_matches_eager(device):
-    q, cache = make(1, 2100, 8, 1, 128, torch.bfloat16, device, 9)
+@pytest.mark.parametrize("q_len,partition", [(9, 0), (9, 192), (100, 0)])
+def test_replay_matches_eager(device, q_len, partition):
+    q, cache = make(1, 2100, 8, 1, 128, torch.bfloat16, device, q_len)
+    assert ops.attend_kernel(q, cache, partition=partition) == ("mfma" if (q_len, partition) == (9, 0) else "tiles")
     out = torch.empty_like(q)
-    ws = torch.zeros(ops.attend_workspace_bytes(q, cache, 2100), dtype=torch.uint8, device=device)
-    args = dict(max_seqlen=2100, seqlen_bias=2100, causal=True, workspace=ws)
+    ws = torch.zeros(ops.attend_workspace_bytes(q, cache, 2100, partition), dtype=torch.uint8, device=device)
+    args = dict(max_seqlen=2100, seqlen_bias=2100, causal=True, workspace=ws, partition=partition)
     want = ops.decode_attention(q, cache, **args)
     graph = torch.cuda.CUDAGraph()
     with torch.cuda.graph(graph):
