@@ -1612,24 +1612,34 @@ static int64_t row_work_per_key(const hexkv_attend_params *p) {
   return heads * p->head_dim * (use_mfma(p, G) ? 3 : 8);  // eighths: the MFMA kernel's cost less
 }
 
+// 128-row tiles of every (sequence, KV head) pair.
+static int64_t tile_count(const hexkv_attend_params *p) {
+  const int64_t rows = static_cast<int64_t>(p->q_len) * (p->q_heads / p->kv_heads);
+  const int64_t per = tile_rows(rows);
+  return static_cast<int64_t>(p->batch) * p->kv_heads * ((rows + per - 1) / per);
+}
+
 static bool rows_lead(const hexkv_attend_params *p) {
   const int group = p->q_heads / p->kv_heads;
   const int64_t segments = static_cast<int64_t>(p->batch) * p->q_len * (p->q_heads / kernel_group(group));
   const int64_t parts = (static_cast<int64_t>(p->max_seqlen) + 127) / 128;
   if (segments * parts <= kRowItems && row_work_per_key(p) * p->max_seqlen <= 8 * kRowWork) return true;
-  const int64_t per = tile_rows(static_cast<int64_t>(p->q_len) * group);
-  const int64_t tiles = static_cast<int64_t>(p->batch) * p->kv_heads * ((static_cast<int64_t>(p->q_len) * group + per - 1) / per);
-  return parts <= 1 && segments <= kFewRows * tiles;
+  return parts <= 1 && segments <= kFewRows * tile_count(p);
 }
 
 // Whether a call runs the query-tile kernel (hexkv_prefill.hip): several
 // query rows per sequence, AUTO, 16-bit data of head_dim 64 or 128, too many
 // rows and keys for the per-row kernels.  An explicit VALU or MFMA request
 // keeps the per-row kernel it names; an explicit partition keeps the tiles it
-// is meant for.
+// is meant for, but for more workgroups than one launch holds (2^32 lanes in
+// x; the per-row kernels' grid has three dimensions).
+static int tile_partition(const hexkv_attend_params *p);
+
 static bool use_tiles(const hexkv_attend_params *p) {
-  return p->q_len > 1 && p->kernel == HEXKV_KERNEL_AUTO && tiles_support(p->dtype, p->head_dim) &&
-         (p->partition > 0 || !rows_lead(p));
+  if (p->q_len <= 1 || p->kernel != HEXKV_KERNEL_AUTO || !tiles_support(p->dtype, p->head_dim)) return false;
+  if (p->partition == 0 && rows_lead(p)) return false;
+  const int64_t part = tile_partition(p);
+  return tile_count(p) * std::max<int64_t>(1, (p->max_seqlen + part - 1) / part) < INT64_C(1) << 24;
 }
 
 // Partition size of a tile call: all keys in one partition unless splitting
@@ -1647,9 +1657,7 @@ static bool use_tiles(const hexkv_attend_params *p) {
 static int tile_partition(const hexkv_attend_params *p) {
   const int per_row = base_partition(p);
   if (p->partition > 0) return per_row;
-  const int64_t rows = static_cast<int64_t>(p->q_len) * (p->q_heads / p->kv_heads);
-  const int64_t per = tile_rows(rows);
-  const int64_t tiles = static_cast<int64_t>(p->batch) * p->kv_heads * ((rows + per - 1) / per);
+  const int64_t tiles = tile_count(p);
   const int64_t keys = std::max<int64_t>(p->max_seqlen, 1);
   const double walk = (12.0 + 0.16 * p->head_dim) * static_cast<double>(keys);
   const double row_heads = static_cast<double>(p->batch) * p->q_len * p->q_heads;

@@ -419,8 +419,8 @@ int launch_tiles(TileArgs a, int dtype, int head_dim, int64_t batch, hipStream_t
   const int64_t rows = static_cast<int64_t>(a.q_len) * a.group;
   const int64_t per = tile_rows(rows);
   const int64_t tiles = (rows + per - 1) / per, pairs = batch * a.kv_heads;
-  if (rows > INT32_MAX || pairs * tiles * a.max_parts > INT32_MAX)
-    return fail(HEXKV_ERANGE, "%s: more than 2^31-1 row tiles", what);
+  if (rows > INT32_MAX || pairs * tiles * a.max_parts >= INT64_C(1) << 24)
+    return fail(HEXKV_ERANGE, "%s: 2^24 row tiles or more", what);
   a.pairs = static_cast<int32_t>(pairs);
   a.tiles = static_cast<int32_t>(tiles);
   const dim3 grid(static_cast<unsigned>(pairs * tiles * a.max_parts));

@@ -204,6 +204,15 @@ def test_several_query_rows_take_the_kernel_that_leads(batch, q_len, hq, hkv, d,
     assert names == sorted(names, key=lambda k: k == "tiles")
 
 
+@pytest.mark.parametrize("longest,expect", [(511 * 64, "tiles"), (511 * 64 + 1, "valu")])
+def test_tiles_fill_at_most_one_launch(longest, expect):
+    """32768 tiles times 512 partitions are 2^24 workgroups of 256 lanes, one
+    too many for a grid's first dimension; the per-row kernels take them."""
+    p = _lib.AttendParams(dtype=_lib.HEXKV_F16, batch=1024, q_len=2, q_heads=32, kv_heads=32, head_dim=64,
+                          capacity=longest, max_seqlen=longest, softmax_scale=1.0, partition=64)
+    assert _lib.KERNEL_NAMES[_lib.load().hexkv_attend_kernel(ctypes.byref(p))] == expect
+
+
 def test_attend_kernel_rejects_bad_geometry():
     p = _lib.AttendParams()
     p.q_heads, p.kv_heads = 6, 4
