@@ -1642,8 +1642,8 @@ static bool use_tiles(const hexkv_attend_params *p) {
   return tile_count(p) * std::max<int64_t>(1, (p->max_seqlen + part - 1) / part) < INT64_C(1) << 24;
 }
 
-// Partition size of a tile call: all keys in one partition unless splitting
-// them pays for the merge.  A tile walks its keys at c = 12 + 0.16 D ns each
+// Partitions of a tile call (before their size is rounded up): one unless
+// splitting the keys pays for the merge.  A tile walks its keys at c = 12 + 0.16 D ns each
 // (one workgroup a slot, 512 slots), and P partitions cost every (row, head)
 // 1.3 + 0.0034 D P ns in partials and the merge launch (fitted on MI355X over
 // 40-4096 rows, 0-4000 earlier keys and four geometries).  The best P is the
@@ -1654,25 +1654,45 @@ static bool use_tiles(const hexkv_attend_params *p) {
 // 1000 keys 40.6 instead of 67.5; 40 rows over 4000 keys 24 (106 unsplit).
 // Never below the per-row kernels' partition, so no call needs more workspace
 // than it did with one.
-static int tile_partition(const hexkv_attend_params *p) {
-  const int per_row = base_partition(p);
-  if (p->partition > 0) return per_row;
+static int64_t tile_parts(const hexkv_attend_params *p) {
   const int64_t tiles = tile_count(p);
   const int64_t keys = std::max<int64_t>(p->max_seqlen, 1);
   const double walk = (12.0 + 0.16 * p->head_dim) * static_cast<double>(keys);
   const double row_heads = static_cast<double>(p->batch) * p->q_len * p->q_heads;
   const double piece = 0.0034 * p->head_dim * row_heads;
   int64_t parts = std::min<int64_t>(512 / std::max<int64_t>(1, tiles), std::llround(std::sqrt(walk / std::max(piece, 1.0))));
-  if (parts < 2 || walk / parts + 1.3 * row_heads + piece * parts >= walk) parts = 1;
+  return parts < 2 || walk / parts + 1.3 * row_heads + piece * parts >= walk ? 1 : parts;
+}
+
+static int tile_partition(const hexkv_attend_params *p) {
+  const int per_row = base_partition(p);
+  if (p->partition > 0) return per_row;
+  const int64_t keys = std::max<int64_t>(p->max_seqlen, 1), parts = tile_parts(p);
   const int64_t part = (keys + parts * 64 - 1) / (parts * 64) * 64;
   return static_cast<int>(std::max<int64_t>(part, per_row));
 }
 
-// The partition whose need the size queries report: never above the one a
-// call runs with, so a workspace sized for the longest step of a loop (and a
-// saved size) serves its shorter ones wherever choose_partition's lines lie.
-static int sizing_partition(const hexkv_attend_params *p) {
-  return use_tiles(p) ? tile_partition(p) : base_partition(p);
+// Partitions per row the size query answers for: at least those the call runs
+// with (choose_partition never takes more than base_partition), and for calls
+// that choose between the tiles and the per-row kernels at least those of
+// every shorter call too, so a workspace sized for the longest chunk of a
+// prompt serves the others.  There rounding the partition up to 64 positions
+// drops a part at some lengths, and the tiles may take no split at all where
+// shorter calls, on the per-row kernels, have several: the bound is the parts
+// before rounding (which only grow with the keys; partitions hold 128
+// positions or more) and those of the longest per-row call, whose partitions
+// hold 128.  A row kernel's own count is not monotone, where base_partition
+// doubles.
+static int64_t sizing_parts(const hexkv_attend_params *p) {
+  const int64_t own = std::max<int64_t>(1, (p->max_seqlen + base_partition(p) - 1) / base_partition(p));
+  if (p->work_items_dev) return std::max<int64_t>(1, p->work_max_parts);
+  if (p->q_len <= 1 || p->kernel != HEXKV_KERNEL_AUTO || !tiles_support(p->dtype, p->head_dim) || p->partition > 0)
+    return own;
+  const int64_t pieces = std::max<int64_t>(1, (static_cast<int64_t>(p->max_seqlen) + 127) / 128);
+  const int64_t segments = std::max<int64_t>(1, static_cast<int64_t>(p->batch) * p->q_len * (p->q_heads / kernel_group(p->q_heads / p->kv_heads)));
+  const int64_t longest = std::min(kRowItems / segments * 128, 8 * kRowWork / std::max<int64_t>(1, row_work_per_key(p)));
+  const int64_t row_parts = std::min(pieces, std::max<int64_t>(1, (longest + 127) / 128));
+  return use_tiles(p) ? std::max(row_parts, std::min(tile_parts(p), pieces)) : std::max(row_parts, own);
 }
 
 static int partition_of(const hexkv_attend_params *p) {
@@ -1694,13 +1714,14 @@ constexpr int64_t kCounterWords = HEXKV_ATTEND_COUNTER_BYTES / sizeof(uint64_t);
 // Workspace: the arrival counters, then the partial outputs
 // [rows][q_heads][max_parts][D], then their (max, sum) pairs
 // [rows][q_heads][max_parts][2], all fp32.
-static size_t workspace_bytes(const hexkv_attend_params *p, int part) {
-  const int64_t max_parts = max_parts_of(p, part);
+static size_t parts_bytes(const hexkv_attend_params *p, int64_t max_parts) {
   if (max_parts <= 1) return 0;
   const int64_t rows = static_cast<int64_t>(p->batch) * p->q_len;
   return HEXKV_ATTEND_COUNTER_BYTES +
          static_cast<size_t>(rows * p->q_heads * max_parts * (p->head_dim + 2)) * sizeof(float);
 }
+
+static size_t workspace_bytes(const hexkv_attend_params *p, int part) { return parts_bytes(p, max_parts_of(p, part)); }
 
 static int validate(const hexkv_attend_params *p) {
   if (!p) return fail(HEXKV_EINVAL, "hexkv_attend: null params");
@@ -2265,7 +2286,7 @@ extern "C" size_t hexkv_attend_workspace_bytes(const hexkv_attend_params *p) {
   if (!p || p->q_heads < 1 || p->kv_heads < 1 || p->q_heads % p->kv_heads || p->q_len < 1 ||
       p->batch < 0 || p->max_seqlen < 0)
     return 0;
-  return workspace_bytes(p, sizing_partition(p));
+  return parts_bytes(p, sizing_parts(p));
 }
 
 extern "C" int hexkv_attend_kernel(const hexkv_attend_params *p) {

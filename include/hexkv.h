@@ -268,8 +268,12 @@ typedef struct hexkv_attend_params {
   int32_t *lengths_out_dev;
 } hexkv_attend_params;
 
-/* Workspace bytes hexkv_attend needs for these parameters (0 when one
- * partition covers every sequence).  The workspace is scratch (partial
+/* Workspace bytes that serve hexkv_attend for these parameters (0 when one
+ * partition covers every sequence).  For q_len > 1 with kernel and partition
+ * 0 (16-bit, head_dim 64 or 128) they also serve every shorter max_seqlen.
+ * Otherwise a shorter call can need a little more, since the library's
+ * partition grows with the call: take the maximum over a loop's steps (a
+ * workspace that fits neither is refused).  The workspace is scratch (partial
  * outputs of the split-K merge) behind HEXKV_ATTEND_COUNTER_BYTES of
  * arrival counters, which single-launch merges (work_xcds > 0) use and
  * leave zero: zero the workspace once after allocating it.  Calls sharing

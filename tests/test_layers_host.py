@@ -4,6 +4,7 @@ for layers whose tensors overlap."""
 import ctypes
 
 import pytest
+import torch
 
 from hexgen2_amd import _lib
 
@@ -75,8 +76,8 @@ def test_layers_independent(change, free):
 @pytest.mark.parametrize("dtype,hq,hkv,d", [(0, 32, 4, 64), (0, 32, 32, 128), (1, 8, 1, 128), (1, 32, 8, 128)])
 @pytest.mark.parametrize("batch", [1, 8, 64])
 def test_workspace_sizes_follow_the_base_partition(dtype, hq, hkv, d, batch):
-    """A decode loop's workspace, sized for its longest step, covers the
-    shorter ones up to where the 128-position rule itself doubles."""
+    """Decode rows: the size of the call's own partitions of 128, 256 or 512
+    positions (not monotone where they double)."""
     lib = _lib.load()
     group = next(g for g in (8, 4, 2, 1) if (hq // hkv) % g == 0)
     for longest in (129, 1024, 1025, 1100, 2048, 4096):
@@ -87,3 +88,33 @@ def test_workspace_sizes_follow_the_base_partition(dtype, hq, hkv, d, batch):
                               capacity=longest, max_seqlen=longest)
         need = _lib.ATTEND_COUNTER_BYTES + batch * hq * parts * (d + 2) * 4 if parts > 1 else 0
         assert lib.hexkv_attend_workspace_bytes(p) == need
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="calls whose workspace fits would run on made-up addresses")
+@pytest.mark.parametrize("dtype,hq,hkv,d", [(0, 32, 4, 64), (0, 32, 32, 128), (1, 8, 1, 128), (1, 32, 8, 128),
+                                            (0, 12, 12, 64), (1, 1, 1, 64)])
+@pytest.mark.parametrize("batch,q_len", [(1, 2), (1, 8), (3, 8), (1, 40), (2, 128), (1, 700), (16, 5), (1, 8192)])
+def test_a_longer_calls_workspace_serves_shorter_chunks(dtype, hq, hkv, d, batch, q_len):
+    """Several query rows: the size never falls as the keys grow, and no call
+    needs more than it (nor more than the per-row kernels' partitions did)."""
+    lib = _lib.load()
+    group = next(g for g in (8, 4, 2, 1) if (hq // hkv) % g == 0)
+    last = 0
+    for n in sorted({*range(q_len, 9000, 61), *(128 * i + j for i in range(1, 70) for j in (0, 1)), 65536}):
+        if n < q_len:
+            continue
+        p = _lib.AttendParams(dtype=dtype, batch=batch, q_len=q_len, q_heads=hq, kv_heads=hkv, head_dim=d, causal=1,
+                              softmax_scale=1.0, q=256, cache=256, out=256, capacity=n, max_seqlen=n, seqlen_bias=n,
+                              q_batch_stride=q_len * hq * d, q_row_stride=hq * d, out_batch_stride=q_len * hq * d,
+                              out_row_stride=hq * d, cache_batch_stride=n * 2 * hkv * d, cache_pos_stride=2 * hkv * d,
+                              cache_kv_stride=hkv * d)
+        need = lib.hexkv_attend_workspace_bytes(p)
+        assert need >= last, n
+        last = need
+        want = batch * q_len * (hq // group) * ((n + 1) // 2) // 2048
+        part = next((s for s in (128, 256) if s >= want), 512)
+        per_row = _lib.ATTEND_COUNTER_BYTES + batch * q_len * hq * -(-n // part) * (d + 2) * 4
+        for size in (need, per_row):
+            # a workspace that is large enough is then refused for its alignment
+            rc = lib.hexkv_attend(p, 8, size, None)
+            assert rc != _lib.HEXKV_EWORKSPACE and rc != 0, (n, size)
