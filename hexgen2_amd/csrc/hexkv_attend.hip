@@ -2613,9 +2613,9 @@ extern "C" int hexkv_attend_noalloc(const hexkv_attend_params *p, hexkv_stream_t
   const char *what = "hexkv_attend_noalloc";
   int rc = validate(p);
   if (rc != HEXKV_OK || p->batch == 0) return rc;
-  // The limit is the need at the base partition, whichever kernel and
-  // partition run (none needs more), so it does not move with their rules.
-  const size_t limit_need = workspace_bytes(p, base_partition(p));
+  // What the size query answers for decode rows (choose_partition's need is
+  // never above it); a tile call's own need, often none.
+  const size_t limit_need = workspace_bytes(p, use_tiles(p) ? partition_of(p) : base_partition(p));
   if (limit_need > HEXKV_NOALLOC_SCRATCH_BYTES)
     return fail(HEXKV_EWORKSPACE,
                 "%s: this call needs %zu bytes of split-K workspace, above the %u-byte static scratch "

@@ -415,8 +415,8 @@ int hexkv_attend_plan_layers(const hexkv_attend_params *p, const int32_t *lens, 
  * HEXKV_NOALLOC_SCRATCH_BYTES (32 MiB) that the library holds on each GPU it
  * runs on until the process ends.  The call allocates nothing (no hipMalloc,
  * no library allocation); the caller still passes q, the cache and out.
- * Returns HEXKV_EWORKSPACE when hexkv_attend_workspace_bytes(p) exceeds the
- * array.  The array's address on a device is looked up on that device's
+ * Returns HEXKV_EWORKSPACE when the call's partials exceed the array (never
+ * when hexkv_attend_workspace_bytes(p) fits it).  The array's address on a device is looked up on that device's
  * first call (the stream's device; the current device for the null stream).
  * Calls on one GPU share its array, which keeps the last call's contents:
  * calls that overlap on one GPU (different streams, no ordering) race.

@@ -108,3 +108,16 @@ def test_noalloc_refuses_beyond_scratch(device):
     out = torch.empty_like(q)
     with pytest.raises(ValueError, match="static scratch"):
         ops.decode_attention_noalloc(q, cache, out, max_seqlen=8192, seqlen_bias=8192, partition=128)
+
+
+@pytest.mark.parametrize("q_len,past", [(2048, 0), (300, 4000), (9, 100)])
+def test_noalloc_takes_several_query_rows_by_what_they_need(device, q_len, past):
+    """A prompt whose tiles need no partials runs, whatever the per-row
+    kernels' partitions would have needed (137 MB for the first)."""
+    n = past + q_len
+    g = torch.Generator(device=device).manual_seed(q_len)
+    q = torch.randn((1, q_len, 32, 128), generator=g, device=device).half()
+    cache = torch.randn((1, n, 2, 8, 128), generator=g, device=device).half()
+    out = torch.empty_like(q)
+    ops.decode_attention_noalloc(q, cache, out, max_seqlen=n, seqlen_bias=n)
+    assert torch.equal(out, ops.decode_attention(q, cache, max_seqlen=n, seqlen_bias=n))
