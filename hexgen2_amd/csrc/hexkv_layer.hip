@@ -435,17 +435,57 @@ static void dispatch_linear(const LinearArgs &a, int rows, int dtype, hipStream_
   }
 }
 
-// The checks that every norm_linear_kernel launch shares.
-static int check_linear(const NormArgs &a, const void *weight, int rows, int es, const char *what) {
-  if (a.h_out && (a.h_out == a.h || a.h_out == a.y)) return fail(HEXKV_EINVAL, "%s: h_out must not be h or y", what);
+// `n` rows of `bytes` each, `stride` bytes apart.
+struct Rows {
+  const void *at;
+  int64_t n, stride, bytes;
+  bool same_as(const Rows &o) const { return at == o.at && (n == 1 || stride == o.stride); }
+};
+
+// Whether two sets of rows share a byte.
+static bool meet(const Rows &a, const Rows &b) {
+  if (!a.at || !b.at || a.n < 1 || b.n < 1) return false;
+  const int64_t a0 = reinterpret_cast<intptr_t>(a.at), b0 = reinterpret_cast<intptr_t>(b.at);
+  if (a0 + (a.n - 1) * a.stride + a.bytes <= b0 || b0 + (b.n - 1) * b.stride + b.bytes <= a0) return false;
+  for (int64_t i = 0; i < a.n; ++i) {
+    // rows j of b that start below this row's end and end above its start
+    const int64_t lo = a0 + i * a.stride - b0 - b.bytes + 1, hi = a0 + i * a.stride + a.bytes - 1 - b0;
+    if (hi < 0) continue;
+    if (b.stride == 0 || b.n == 1) {
+      if (lo <= 0) return true;
+      continue;
+    }
+    const int64_t first = lo <= 0 ? 0 : (lo + b.stride - 1) / b.stride;
+    if (first < b.n && first * b.stride <= hi) return true;
+  }
+  return false;
+}
+
+static int refuse_overlap(const char *out, const char *in, const char *what) {
+  return fail(HEXKV_EINVAL, "%s: %s overlaps %s, which other workgroups read or write meanwhile", what, out, in);
+}
+
+// The checks that every norm_linear_kernel launch shares.  Every workgroup
+// reads all of h and y, and workgroup 0 stores their sum, while others store
+// the products: no output may share a byte with an input or another output.
+static int check_linear(const NormArgs &a, const Rows &weight, const Rows (&outs)[2], int rows, int es, const char *what) {
   if (a.h_stride < 0 || a.y_stride < 0 || a.h_out_stride < 0) return fail(HEXKV_EINVAL, "%s: negative stride", what);
   const int64_t vec = 16 / es;
   if (rows > kLinearRows || static_cast<int64_t>(rows) * a.hidden * es > kLinearLds)
     return fail(HEXKV_EUNSUPPORTED, "%s: at most %d rows and %lld bytes of them", what, kLinearRows,
                 static_cast<long long>(kLinearLds));
   if (a.hidden % vec || a.h_stride % vec || a.y_stride % vec || a.h_out_stride % vec || !aligned16(a.h) ||
-      !aligned16(a.y) || !aligned16(a.h_out) || !aligned16(a.weight) || !aligned16(weight))
+      !aligned16(a.y) || !aligned16(a.h_out) || !aligned16(a.weight) || !aligned16(weight.at))
     return fail(HEXKV_EUNSUPPORTED, "%s: rows must be 16-byte aligned and a multiple of 16 bytes", what);
+  const int64_t row = static_cast<int64_t>(a.hidden) * es;
+  const Rows in[] = {{a.h, rows, a.h_stride * es, row}, {a.y, rows, a.y_stride * es, row}, {a.weight, 1, row, row}, weight};
+  const Rows out[] = {{a.h_out, rows, a.h_out_stride * es, row}, outs[0], outs[1]};
+  if (a.h_out && rows > 1 && a.h_out_stride < a.hidden) return fail(HEXKV_EINVAL, "%s: h_out's rows overlap", what);
+  for (const Rows &o : out)
+    for (const Rows &i : in)
+      if (meet(o, i)) return refuse_overlap("an output", "an input", what);
+  if (meet(out[0], out[1]) || meet(out[0], out[2]) || meet(out[1], out[2]))
+    return refuse_overlap("an output", "another", what);
   return HEXKV_OK;
 }
 
@@ -465,7 +505,9 @@ extern "C" int hexkv_norm_linear(const void *h, int64_t h_stride, const void *y,
   if (!h || !weight || !out) return fail(HEXKV_EINVAL, "%s: null tensor", what);
   const LinearArgs a{NormArgs{h, y, norm_weight, h_out, nullptr, h_stride, y_stride, h_out_stride, hidden, eps},
                      weight, out, n, RopeArgs{}};
-  const int bad = check_linear(a.norm, weight, rows, es, what);
+  const int64_t w_bytes = (glu ? 2 : 1) * static_cast<int64_t>(n) * hidden * es, out_row = static_cast<int64_t>(n) * es;
+  const int bad = check_linear(a.norm, Rows{weight, 1, w_bytes, w_bytes}, {Rows{out, rows, out_row, out_row}, Rows{}},
+                               rows, es, what);
   if (bad != HEXKV_OK) return bad;
   hipStream_t s = static_cast<hipStream_t>(stream);
   if (glu) dispatch_linear<kLinearGlu>(a, rows, dtype, s);
@@ -495,7 +537,10 @@ extern "C" int hexkv_norm_rope_linear(const void *h, int64_t h_stride, const voi
   const LinearArgs a{NormArgs{h, y, norm_weight, h_out, nullptr, h_stride, y_stride, h_out_stride, hidden, eps},
                      weight, nullptr, static_cast<int32_t>(units),
                      RopeArgs{nullptr, q, kv, inv_freq_dev, positions_dev, 0, q_heads, kv_heads, head_dim, seqlen, offset}};
-  const int bad = check_linear(a.norm, weight, rows, es, what);
+  const int64_t w_bytes = 2 * units * hidden * es, q_row = static_cast<int64_t>(q_heads) * head_dim * es;
+  const int64_t kv_row = 2 * static_cast<int64_t>(kv_heads) * head_dim * es;
+  const int bad = check_linear(a.norm, Rows{weight, 1, w_bytes, w_bytes},
+                               {Rows{q, rows, q_row, q_row}, Rows{kv, rows, kv_row, kv_row}}, rows, es, what);
   if (bad != HEXKV_OK) return bad;
   dispatch_linear<kLinearRope>(a, rows, dtype, static_cast<hipStream_t>(stream));
   return check_launch(what);
@@ -515,6 +560,17 @@ extern "C" int hexkv_add_rms_norm(const void *h, int64_t h_stride, const void *y
   if (rows == 0) return HEXKV_OK;
   if (!h || !weight || !out) return fail(HEXKV_EINVAL, "%s: null tensor", what);
   const NormArgs a{h, y, weight, h_out, out, h_stride, y_stride, h_out_stride, hidden, eps};
+  // A workgroup reads its own row and the weight, and each lane writes the
+  // elements it read: in place row for row, but over no other row.
+  const int64_t row = static_cast<int64_t>(hidden) * es;
+  const Rows r_h{h, rows, h_stride * es, row}, r_y{y, rows, y_stride * es, row}, r_w{weight, 1, row, row};
+  const Rows r_sum{h_out, rows, h_out_stride * es, row}, r_out{out, rows, row, row};
+  if (h_out && rows > 1 && h_out_stride < hidden) return fail(HEXKV_EINVAL, "%s: h_out's rows overlap", what);
+  for (const Rows &o : {r_sum, r_out}) {
+    if (meet(o, r_w)) return refuse_overlap("an output", "the weight", what);
+    for (const Rows &i : {r_h, r_y, r_sum})
+      if (!o.same_as(i) && meet(o, i)) return refuse_overlap("an output", "rows of another tensor", what);
+  }
   const int64_t vec = 16 / es;
   const bool vec16 = hidden % vec == 0 && h_stride % vec == 0 && y_stride % vec == 0 && h_out_stride % vec == 0 &&
                      aligned16(h) && aligned16(y) && aligned16(h_out) && aligned16(weight) && aligned16(out);
@@ -545,6 +601,13 @@ extern "C" int hexkv_rope_split(const void *qkv, int64_t qkv_stride, const float
     return fail(HEXKV_ERANGE, "%s: position offset %d", what, offset);
   if (rows == 0) return HEXKV_OK;
   if (!qkv || !inv_freq_dev || !q || !kv) return fail(HEXKV_EINVAL, "%s: null tensor", what);
+  // One row may be split where it stands: a lane writes what it read.
+  const int64_t q_row = static_cast<int64_t>(q_heads) * head_dim * es, kv_row = row * es - q_row;
+  const Rows r_in{qkv, rows, qkv_stride * es, row * es}, r_q{q, rows, q_row, q_row}, r_kv{kv, rows, kv_row, kv_row};
+  if ((!(rows == 1 && q == qkv) && meet(r_q, r_in)) ||
+      (!(rows == 1 && kv == static_cast<const char *>(qkv) + q_row) && meet(r_kv, r_in)))
+    return refuse_overlap("q or kv", "qkv", what);
+  if (meet(r_q, r_kv)) return refuse_overlap("q", "kv", what);
   const RopeArgs a{qkv, q, kv, inv_freq_dev, positions_dev, qkv_stride, q_heads, kv_heads, head_dim, seqlen, offset};
   const int vec = 16 / es;
   const bool vec16 = (head_dim / 2) % vec == 0 && qkv_stride % vec == 0 && aligned16(qkv) && aligned16(q) && aligned16(kv);
@@ -568,6 +631,12 @@ extern "C" int hexkv_silu_mul(const void *gate_up, void *out, int64_t rows, int 
   if (width < 1 || width > 1 << 23) return fail(HEXKV_EINVAL, "%s: width %d outside [1, 2^23]", what, width);
   if (rows == 0) return HEXKV_OK;
   if (!gate_up || !out) return fail(HEXKV_EINVAL, "%s: null tensor", what);
+  // One row's result may take the place of its gate or its up half.
+  const int64_t half = static_cast<int64_t>(width) * es;
+  const char *gate = static_cast<const char *>(gate_up);
+  if (!(rows == 1 && (out == gate || out == gate + half)) &&
+      meet(Rows{out, rows, half, half}, Rows{gate_up, rows, 2 * half, 2 * half}))
+    return refuse_overlap("out", "gate_up", what);
   const bool vec16 = width % (16 / es) == 0 && aligned16(gate_up) && aligned16(out);
   hipStream_t s = static_cast<hipStream_t>(stream);
   switch (dtype) {

@@ -612,18 +612,21 @@ void *hexkv_ipc_dlpack(void *base, uint64_t offset, int ndim, const int64_t *sha
 /* ------------------------------------------------- decoder layer steps ---
  * The steps between a decoder layer's matrix products, one launch each (the
  * reference runs them as separate tensor operations).  Strides are in
- * elements, rows of `out`, `q` and `kv` are contiguous, below 2^24 rows. */
+ * elements, rows of `out`, `q` and `kv` are contiguous, below 2^24 rows.
+ * Workgroups run in any order, so outputs that overlap inputs or each other
+ * are refused (HEXKV_EINVAL) but where a call says they may. */
 
 /* out[r] = rms_norm(h[r] + y[r]) * weight (rms_norm.py:13-15; the residual
- * sum of modules/block.py:112-175).  y NULL: no sum.  h_out (may be h, or
- * NULL) receives the sum rounded to the data type. */
+ * sum of modules/block.py:112-175).  y NULL: no sum.  h_out (or NULL)
+ * receives the sum rounded to the data type.  h_out and out may be h or y,
+ * row for row. */
 int hexkv_add_rms_norm(const void *h, int64_t h_stride, const void *y, int64_t y_stride, void *h_out,
                        int64_t h_out_stride, const void *weight, void *out, int64_t rows, int hidden,
                        float eps, int dtype, hexkv_stream_t stream);
 
 /* out = x W^T for up to 2 tokens, W [n][hidden] (contiguous), one launch:
  * x = h, or with norm_weight rms_norm(h + y) * norm_weight (y may be NULL),
- * the sum also written to h_out (NULL, or neither h nor y).  With glu W is
+ * the sum also written to h_out (or NULL).  With glu W is
  * [2 n][hidden] and out[i] = silu(x W[i]) * (x W[n + i]), rounded once.
  * HEXKV_EUNSUPPORTED above 2 rows or 64 KiB of them, or when hidden, strides
  * or addresses are not multiples of 16 bytes. */
@@ -642,12 +645,14 @@ int hexkv_norm_rope_linear(const void *h, int64_t h_stride, const void *y, int64
 /* Rows [q heads | k heads | v heads] of head_dim elements (qkv_stride apart)
  * into q [rows][q_heads][head_dim] and kv [rows][2][kv_heads][head_dim], q
  * and k rotated (GPT-NeoX halves) by position * inv_freq_dev[j].  Row r is
- * position r % seqlen + offset, or positions_dev[r / seqlen] when given. */
+ * position r % seqlen + offset, or positions_dev[r / seqlen] when given.  One
+ * row may be split in place (q at qkv, kv behind it). */
 int hexkv_rope_split(const void *qkv, int64_t qkv_stride, const float *inv_freq_dev,
                      const int32_t *positions_dev, int offset, void *q, void *kv, int64_t rows, int seqlen,
                      int q_heads, int kv_heads, int head_dim, int dtype, hexkv_stream_t stream);
 
-/* out[r][i] = silu(gate_up[r][i]) * gate_up[r][width + i] (mlp.py:63-87). */
+/* out[r][i] = silu(gate_up[r][i]) * gate_up[r][width + i] (mlp.py:63-87).
+ * One row's out may be either half of gate_up. */
 int hexkv_silu_mul(const void *gate_up, void *out, int64_t rows, int width, int dtype, hexkv_stream_t stream);
 
 #ifdef __cplusplus

@@ -1,6 +1,7 @@
 """Planning of lists that several layers share, on the host: one layer gets
-the one-layer rules, several a chunk that every kernel accepts; and the check
-for layers whose tensors overlap."""
+the one-layer rules, several a chunk that every kernel accepts; the checks for
+tensors that overlap, of layers and of the steps between products; and the
+workspace sizes."""
 import ctypes
 
 import pytest
@@ -118,3 +119,60 @@ def test_a_longer_calls_workspace_serves_shorter_chunks(dtype, hq, hkv, d, batch
             # a workspace that is large enough is then refused for its alignment
             rc = lib.hexkv_attend(p, 8, size, None)
             assert rc != _lib.HEXKV_EWORKSPACE and rc != 0, (n, size)
+
+
+def _linear(lib, h, y, h_out, norm, w, out, rows=2, hidden=64, n=16, glu=0, stride=64):
+    return lib.hexkv_norm_linear(h, stride, y, stride, h_out, stride, norm, 1e-5, w, out, rows, hidden, n, glu, 0, None)
+
+
+def _rope_linear(lib, h, y, h_out, norm, w, q, kv, rows=2):
+    return lib.hexkv_norm_rope_linear(h, 64, y, 64, h_out, 64, norm, 1e-5, w, 0x900000, None, 0, q, kv, rows, rows, 64,
+                                      4, 2, 16, 0, None)
+
+
+H, Y, S, N, W, O, K = (0x100000 * i for i in range(1, 8))  # 2 rows of 64 float16 elements: 256 bytes; W 8192 at most
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="accepted calls would run on made-up addresses")
+@pytest.mark.parametrize("clash,call", [
+    (False, lambda l: _linear(l, H, Y, S, N, W, O)),
+    (True, lambda l: _linear(l, H, Y, H, N, W, O)),           # the sum over h
+    (True, lambda l: _linear(l, H, Y, H + 128, N, W, O)),     # over h's second row
+    (True, lambda l: _linear(l, H, Y, S, N, W, H)),           # out over h
+    (True, lambda l: _linear(l, H, Y, S, N, W, Y, n=64)),     # out over y, as large
+    (True, lambda l: _linear(l, H, None, None, N, W, H + 240)),
+    (False, lambda l: _linear(l, H, None, None, N, W, H + 256)),
+    (False, lambda l: _linear(l, H, None, None, N, W, H + 128, rows=1)),
+    (True, lambda l: _linear(l, H, Y, S, N, W, S + 128)),     # out over the sum
+    (True, lambda l: _linear(l, H, Y, S, N, W, N)),           # out over the norm's weight
+    (True, lambda l: _linear(l, H, Y, S, N, W, W + 16 * 128 - 16)),
+    (False, lambda l: _linear(l, H, Y, S, N, W, W + 16 * 128)),
+    (True, lambda l: _linear(l, H, Y, S, N, W, W + 16 * 128, glu=1)),
+    (False, lambda l: _linear(l, H, H + 128, H + 256, N, W, O, stride=192)),  # rows of one buffer, side by side
+    (True, lambda l: _linear(l, H, H + 128, H + 192, N, W, O, stride=192)),
+    (False, lambda l: _rope_linear(l, H, Y, S, N, W, O, K)),
+    (True, lambda l: _rope_linear(l, H, Y, S, N, W, H, K)),
+    (True, lambda l: _rope_linear(l, H, Y, S, N, W, O, Y + 16)),
+    (True, lambda l: _rope_linear(l, H, Y, S, N, W, O, O + 128)),
+    (True, lambda l: _rope_linear(l, H, Y, S, N, W, W + 8 * 16 * 128 - 16, K)),
+    (False, lambda l: l.hexkv_add_rms_norm(H, 64, Y, 64, H, 64, N, Y, 2, 64, 1e-5, 0, None)),   # row for row
+    (True, lambda l: l.hexkv_add_rms_norm(H, 64, Y, 64, H + 128, 64, N, O, 2, 64, 1e-5, 0, None)),
+    (True, lambda l: l.hexkv_add_rms_norm(H, 128, Y, 64, None, 0, N, H, 2, 64, 1e-5, 0, None)),  # h's rows lie apart
+    (False, lambda l: l.hexkv_add_rms_norm(H, 128, Y, 64, None, 0, N, H, 1, 64, 1e-5, 0, None)),
+    (True, lambda l: l.hexkv_add_rms_norm(H, 64, Y, 64, None, 0, N, N, 2, 64, 1e-5, 0, None)),
+    (True, lambda l: l.hexkv_add_rms_norm(H, 0, Y, 64, H, 0, N, O, 2, 64, 1e-5, 0, None)),      # one row for both
+    (False, lambda l: l.hexkv_add_rms_norm(H, 0, Y, 64, None, 0, N, O, 2, 64, 1e-5, 0, None)),
+    (False, lambda l: l.hexkv_rope_split(H, 128, 0x900000, None, 0, O, K, 2, 2, 4, 2, 16, 0, None)),
+    (True, lambda l: l.hexkv_rope_split(H, 128, 0x900000, None, 0, H, K, 2, 2, 4, 2, 16, 0, None)),
+    (False, lambda l: l.hexkv_rope_split(H, 128, 0x900000, None, 0, H, H + 128, 1, 1, 4, 2, 16, 0, None)),
+    (True, lambda l: l.hexkv_rope_split(H, 128, 0x900000, None, 0, O, O + 128, 2, 2, 4, 2, 16, 0, None)),
+    (False, lambda l: l.hexkv_silu_mul(H, H + 128, 1, 64, 0, None)),
+    (True, lambda l: l.hexkv_silu_mul(H, H, 2, 64, 0, None)),
+    (True, lambda l: l.hexkv_silu_mul(H, H + 64, 1, 64, 0, None)),
+    (False, lambda l: l.hexkv_silu_mul(H, H + 512, 2, 64, 0, None))])
+def test_overlapping_outputs_are_refused(clash, call):
+    """Workgroups of the layer steps read whole inputs while others store."""
+    lib = _lib.load()
+    rc = call(lib)
+    assert (rc == _lib.HEXKV_EINVAL) == clash, lib.hexkv_last_error()
+    assert not clash or b"overlap" in lib.hexkv_last_error()
