@@ -414,8 +414,11 @@ def decode_attention(q: torch.Tensor, cache: torch.Tensor, *, max_seqlen: int,
     _require_device(q, cache)
     lib = _lib.load()
     softmax_scale = None if softmax_scale is None else float(softmax_scale)
-    key = (_tensor_geometry(q), _tensor_geometry(cache), _tensor_geometry(out), _tensor_geometry(kv_new),
-           _tensor_geometry(seqlens), bool(causal), softmax_scale, int(partition), kernel)
+    # (the cache's capacity is set per call: a view that grows by a token is one form)
+    shape = cache.shape
+    key = (_tensor_geometry(q), shape[:1] + shape[2:], cache.stride(), cache.dtype, cache.get_device(),
+           _tensor_geometry(out), _tensor_geometry(kv_new), _tensor_geometry(seqlens), bool(causal), softmax_scale,
+           int(partition), kernel)
     if out is None:
         out = q.new_empty(q.shape)
     form = _ATTEND_FORMS.get(key)
@@ -432,7 +435,7 @@ def decode_attention(q: torch.Tensor, cache: torch.Tensor, *, max_seqlen: int,
             p.kv_new = kv_new.data_ptr()
         if seqlens is not None:
             p.seqlens_dev = seqlens.data_ptr()
-        p.seqlen_bias, p.max_seqlen = int(seqlen_bias), int(max_seqlen)
+        p.seqlen_bias, p.max_seqlen, p.capacity = int(seqlen_bias), int(max_seqlen), shape[1]
     work = None
     if lens is not None:
         work = _plan_work(p, lens, q.device, single_launch)  # kept alive until the launch is enqueued
@@ -460,9 +463,9 @@ def decode_attention(q: torch.Tensor, cache: torch.Tensor, *, max_seqlen: int,
 
 
 # decode_attention's checked parameter blocks by what they depend on: every
-# tensor's shape, strides, dtype and device, and the options, never an
-# address.  (block, {max_seqlen: workspace bytes}) each; the addresses and
-# lengths of a call go into a copy.  Building and checking the block anew
+# tensor's shape (but for the cache's capacity), strides, dtype and device, and
+# the options, never an address.  (block, {max_seqlen: workspace bytes}) each;
+# the addresses and lengths of a call go into a copy.  Building and checking the block anew
 # was about 9 of an eager decode layer's 20 us of host time.
 _ATTEND_FORMS: "OrderedDict[tuple, tuple]" = OrderedDict()
 

@@ -56,6 +56,20 @@ def test_kept_blocks_refuse_what_a_first_call_refuses(device):
     assert len(ops._ATTEND_FORMS) <= 64
 
 
+def test_a_growing_view_keeps_one_block(device):
+    """A decode loop over cache views one token longer each step keeps a few
+    blocks, and a kept block admits no length past the view it is called with."""
+    cache = torch.randn(2, 300, 2, 2, 64, device="cuda").half()
+    q = torch.randn(2, 1, 8, 64, device="cuda").half()
+    ops._ATTEND_FORMS.clear()
+    for n in range(200, 300):
+        got = ops.decode_attention(q, cache[:, :n], max_seqlen=n, seqlen_bias=n)
+    assert len(ops._ATTEND_FORMS) == 1
+    assert torch.equal(got, ops.decode_attention(q, cache[:, :299].clone(), max_seqlen=299, seqlen_bias=299))
+    with pytest.raises(ValueError):
+        ops.decode_attention(q, cache[:, :250], max_seqlen=251, seqlen_bias=251)
+
+
 @pytest.mark.parametrize("start,batch,offset,length", [(0, 3, 0, 5), (1, 2, 3, 2), (2, 1, 7, 9), (0, 1, 14, 2), (1, 1, 0, 16)])
 @pytest.mark.parametrize("pad", [0, 8])
 def test_cache_write(device, start, batch, offset, length, pad):
