@@ -1615,8 +1615,7 @@ static int64_t row_work_per_key(const hexkv_attend_params *p) {
 // 128-row tiles of every (sequence, KV head) pair.
 static int64_t tile_count(const hexkv_attend_params *p) {
   const int64_t rows = static_cast<int64_t>(p->q_len) * (p->q_heads / p->kv_heads);
-  const int64_t per = tile_rows(rows);
-  return static_cast<int64_t>(p->batch) * p->kv_heads * ((rows + per - 1) / per);
+  return static_cast<int64_t>(p->batch) * p->kv_heads * ((rows + kTileRows - 1) / kTileRows);
 }
 
 static bool rows_lead(const hexkv_attend_params *p) {

@@ -28,8 +28,9 @@ struct TileArgs {
 // Whether the kernel is compiled for these types and sizes.
 bool tiles_support(int dtype, int head_dim);
 
-// Query rows of one pair (q_len * group of them) per workgroup.
-int tile_rows(int64_t pair_rows);
+// Query rows of one pair (q_len * group of them) per workgroup: 32 for each of
+// its four waves.
+constexpr int kTileRows = 128;
 
 // One launch over every tile (and key partition); a.pairs, a.q_len, a.group
 // and a.max_parts set, a.tiles filled here.

@@ -56,6 +56,7 @@ namespace hexkv {
 
 constexpr int kTileThreads = 256;
 constexpr int kTileWaves = kTileThreads / 64;
+static_assert(kTileRows == 32 * kTileWaves, "32 query rows a wave");
 constexpr float kLowest = -1e30f;   // finite "minus infinity" of the running maximum
 
 typedef short h4 __attribute__((ext_vector_type(4)));
@@ -185,11 +186,11 @@ __device__ __forceinline__ void exact_row(const TileArgs &a, int b, int t, int q
   }
 }
 
-// NKB: 32-key blocks per tile.
-template <typename T, int D, int NKB>
+template <typename T, int D>
 __global__ __launch_bounds__(kTileThreads, 2) void attend_tile_kernel(const TileArgs a) {
   using M = Mma32<T>;
-  constexpr int ROWS = 32 * kTileWaves;   // query rows per workgroup
+  constexpr int ROWS = kTileRows;
+  constexpr int NKB = 2;                  // 32-key blocks per tile
   constexpr int KT = 32 * NKB;            // keys per tile
   constexpr int NJ = D / 16;              // score k-steps
   constexpr int ND = D / 32;              // output blocks of 32 dims
@@ -407,18 +408,15 @@ bool tiles_support(int dtype, int head_dim) {
   return (dtype == HEXKV_F16 || dtype == HEXKV_BF16) && (head_dim == 64 || head_dim == 128);
 }
 
-int tile_rows(int64_t) { return 32 * kTileWaves; }
-
 template <typename T, int D>
 static void launch_tile(const TileArgs &a, dim3 grid, hipStream_t s) {
-  attend_tile_kernel<T, D, 2><<<grid, kTileThreads, 0, s>>>(a);
+  attend_tile_kernel<T, D><<<grid, kTileThreads, 0, s>>>(a);
 }
 
 int launch_tiles(TileArgs a, int dtype, int head_dim, int64_t batch, hipStream_t s, const char *what) {
   if (!tiles_support(dtype, head_dim)) return fail(HEXKV_EUNSUPPORTED, "%s: no tile kernel for head_dim %d", what, head_dim);
   const int64_t rows = static_cast<int64_t>(a.q_len) * a.group;
-  const int64_t per = tile_rows(rows);
-  const int64_t tiles = (rows + per - 1) / per, pairs = batch * a.kv_heads;
+  const int64_t tiles = (rows + kTileRows - 1) / kTileRows, pairs = batch * a.kv_heads;
   if (rows > INT32_MAX || pairs * tiles * a.max_parts >= INT64_C(1) << 24)
     return fail(HEXKV_ERANGE, "%s: 2^24 row tiles or more", what);
   a.pairs = static_cast<int32_t>(pairs);
