@@ -416,7 +416,9 @@ def decode_attention(q: torch.Tensor, cache: torch.Tensor, *, max_seqlen: int,
     softmax_scale = None if softmax_scale is None else float(softmax_scale)
     # (the cache's capacity is set per call: a view that grows by a token is one form)
     shape = cache.shape
-    key = (_tensor_geometry(q), shape[:1] + shape[2:], cache.stride(), cache.dtype, cache.get_device(),
+    if len(shape) != 5:
+        raise ValueError("the cache must be [batch, capacity, 2, kv_heads, head_dim]")
+    key = (_tensor_geometry(q), shape[0], shape[2], shape[3], shape[4], cache.stride(), cache.dtype, cache.get_device(),
            _tensor_geometry(out), _tensor_geometry(kv_new), _tensor_geometry(seqlens), bool(causal), softmax_scale,
            int(partition), kernel)
     if out is None:
