@@ -1597,7 +1597,7 @@ static bool use_mfma(const hexkv_attend_params *p, int G);
 // cost more than the keys it saves.  Lines from 4000 random calls (14
 // geometries of group 1-16, 1-64 sequences, 2-200 rows, up to 16000 keys):
 // by this rule 15 of them take over 1.1 times the per-row kernels' time (at
-// most 1.36), the tile kernel for all of them 1500 (at most 2.1), and the
+// most 1.36) where the tile kernel for all had 1475 such (at most 2.1), and the
 // geometric mean is within 1% of the faster kernel for each.  Tiles and
 // per-row kernel, us: TinyLlama, 16 rows over 100 keys 6.2 and 4.0, 64 over
 // 8000 21.6 and 55.9; Llama-2-7B 16 over 100 7.1 and 4.5, 64 over 1000 22 and
@@ -1626,14 +1626,14 @@ static bool rows_lead(const hexkv_attend_params *p) {
   return parts <= 1 && segments <= kFewRows * tile_count(p);
 }
 
+static int tile_partition(const hexkv_attend_params *p);
+
 // Whether a call runs the query-tile kernel (hexkv_prefill.hip): several
 // query rows per sequence, AUTO, 16-bit data of head_dim 64 or 128, too many
 // rows and keys for the per-row kernels.  An explicit VALU or MFMA request
 // keeps the per-row kernel it names; an explicit partition keeps the tiles it
 // is meant for, but for more workgroups than one launch holds (2^32 lanes in
 // x; the per-row kernels' grid has three dimensions).
-static int tile_partition(const hexkv_attend_params *p);
-
 static bool use_tiles(const hexkv_attend_params *p) {
   if (p->q_len <= 1 || p->kernel != HEXKV_KERNEL_AUTO || !tiles_support(p->dtype, p->head_dim)) return false;
   if (p->partition == 0 && rows_lead(p)) return false;
@@ -1642,10 +1642,11 @@ static bool use_tiles(const hexkv_attend_params *p) {
 }
 
 // Partitions of a tile call (before their size is rounded up): one unless
-// splitting the keys pays for the merge.  A tile walks its keys at c = 12 + 0.16 D ns each
-// (one workgroup a slot, 512 slots), and P partitions cost every (row, head)
-// 1.3 + 0.0034 D P ns in partials and the merge launch (fitted on MI355X over
-// 40-4096 rows, 0-4000 earlier keys and four geometries).  The best P is the
+// splitting the keys pays for the merge.  A tile walks its keys at c = 12 +
+// 0.16 D ns each (one workgroup a slot, 512 slots), and P partitions cost
+// every (row, head) 1.3 + 0.0034 D P ns in partials and the merge launch
+// (fitted on MI355X over 40-4096 rows, 0-4000 earlier keys and four
+// geometries).  The best P is the
 // square root of c keys / (0.0034 D rows heads), and it is taken if its sum is
 // below c keys.  Per call, against 512 workgroups whatever the merge costs:
 // TinyLlama's 512- and 1024-token prompts 14.3 and 24.6 us instead of 27.1
@@ -1688,8 +1689,10 @@ static int64_t sizing_parts(const hexkv_attend_params *p) {
   if (p->q_len <= 1 || p->kernel != HEXKV_KERNEL_AUTO || !tiles_support(p->dtype, p->head_dim) || p->partition > 0)
     return own;
   const int64_t pieces = std::max<int64_t>(1, (static_cast<int64_t>(p->max_seqlen) + 127) / 128);
-  const int64_t segments = std::max<int64_t>(1, static_cast<int64_t>(p->batch) * p->q_len * (p->q_heads / kernel_group(p->q_heads / p->kv_heads)));
-  const int64_t longest = std::min(kRowItems / segments * 128, 8 * kRowWork / std::max<int64_t>(1, row_work_per_key(p)));
+  const int64_t groups = p->q_heads / kernel_group(p->q_heads / p->kv_heads);
+  const int64_t segments = std::max<int64_t>(1, static_cast<int64_t>(p->batch) * p->q_len * groups);
+  const int64_t longest =
+      std::min(kRowItems / segments * 128, 8 * kRowWork / std::max<int64_t>(1, row_work_per_key(p)));
   const int64_t row_parts = std::min(pieces, std::max<int64_t>(1, (longest + 127) / 128));
   return use_tiles(p) ? std::max(row_parts, std::min(tile_parts(p), pieces)) : std::max(row_parts, own);
 }

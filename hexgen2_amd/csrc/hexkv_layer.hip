@@ -199,13 +199,19 @@ __global__ __launch_bounds__(kLayerThreads) void silu_mul_kernel(const T *__rest
 // just the same.
 //
 // Measured on MI355X in fp16, one token, against the norm, the library's
-// product and the SwiGLU as launches of their own: 2048 -> 2560 with norm 4.8
-// and 9.8 us, 2048 -> 2 x 5632 with norm and SwiGLU 10.2 and 19.6, 5632 ->
-// 2048 7.3 and 10.4, 4096 -> 2 x 11008 30.4 and 57.1 (5.9 TB/s), 4096 ->
-// 32000 41.3 and 58.3 (6.3 TB/s); with the heads split and turned in it as
-// well the model call of the head comment goes from 1.48 to 1.41 ms.  Two tokens take 5-25% longer, the
-// library's no longer; with four, norm and 4096 -> 12288 took 27.9 and
-// 23.8, so the line is at two.
+// product and the SwiGLU as launches of their own: 64 -> 64 with norm 2.7 and
+// 4.6 us, 2048 -> 2560 with norm 4.8 and 10.1, 2048 -> 2 x 5632 with norm and
+// SwiGLU 10.0 and 19.3, 5632 -> 2048 7.3 and 10.5, 4096 -> 2 x 14336 36.9 and
+// 40.3 (6.4 TB/s), 4096 -> 32000 with norm 40.3 and 42.8 (6.5 TB/s); with the
+// heads split and turned in it as well the model call of the head comment
+// goes from 1.48 to 1.41 ms.  Two tokens take 5-25% longer, the library's no
+// longer.  Of 110 products of one and two tokens in fp16, bf16 and fp32 (64 to
+// 14336 -> 64 to 128256, plain and with norm) four lose to the library, by
+// 3-9%: 4096 -> 28672 without norm, 4096 -> 32000 with norm and two tokens in
+// fp16 (45.4 and 43.2), 14336 -> 4096 in fp32 without norm (38.4 and 35.2).
+// The line is at two tokens for want of instances beyond: with four, norm and
+// 4096 -> 12288 took 27.9 and 23.8, and three, or the small products where
+// the kernel leads most, were not measured.
 constexpr int kLinearRows = 2;
 constexpr int64_t kLinearLds = INT64_C(64) << 10;  // x in LDS: two workgroups a CU at least
 

@@ -1,5 +1,6 @@
 // Attention of several query rows per sequence (a prompt, or a later chunk
-// of one) over the KV cache: hexkv_attend with q_len > 1.
+// of one) over the KV cache: hexkv_attend with q_len > 1, but for small calls
+// (rows_lead in hexkv_attend.hip).
 //
 // What bounds it: the decode kernels stream a row's keys once per query row,
 // so a prompt of n tokens reads n / 2 times its K and V; a tile of rows that
@@ -10,7 +11,7 @@
 // Measured on MI355X against the decode kernels row by row: Llama-3-8B's
 // 8192-token layer 760-810 us and 16.9 ms, 700 TFLOP/s of the products
 // without the lo halves (1.05 PFLOP/s with them; a library product reaches
-// 1.2), matrix cores 53% and VALU 46% busy, LDS 26%; a Llama-2-7B chunk of
+// 1.2), matrix cores 55% and VALU 48% busy, LDS 27%; a Llama-2-7B chunk of
 // 2 x 611 over 512 keys 55 and 1165 us.
 //
 // Work split: a workgroup (4 waves) takes ROWS of the q_len * group query
@@ -21,7 +22,7 @@
 // tiles meet its K and V in one XCD's L2.  Tiles run from the longest rows
 // down.  When the tiles alone leave CUs idle and the rows are few for their
 // keys (a short chunk over a long past), the keys are cut into partitions
-// merged by combine_kernel as for decode rows (tile_partition).
+// merged by combine_kernel as for decode rows (tile_parts).
 //
 // One wave, 32 query rows (one per lane and half):
 //   S^T = K Q^T   v_mfma_f32_32x32x16, K (A) from LDS, Q (B) in registers:
@@ -35,7 +36,11 @@
 //                 ds_read_b64_tr_b16 in the same order.  Every probability
 //                 enters as hi + lo 16-bit values (about 2^-17 relative for
 //                 bf16; 2^-22 for fp16, or 2^-36 of the row's largest),
-//                 both products exact in fp32.
+//                 both products exact in fp32.  (The accumulators take 16
+//                 products at a time, in fp32: over 2^20 keys of 2^-25 of
+//                 the largest, together 2.7% of the output, they lost a
+//                 fifth to a third of it; at 8192 keys the error against 64 bits is the
+//                 output's own rounding.)
 // A lane's accumulators all belong to its own row, so rescaling and the
 // final division need no exchange.
 //

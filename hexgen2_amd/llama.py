@@ -10,8 +10,12 @@ calls are exactly the reference's: ``_update_kv_cache`` then
 with ``fused_ft_kernel`` the decode steps call
 ``_apply_rotary_single_query_attention`` on unrotated q/k (mha.py:553-571).
 Dense projections use torch (hipBLASLt), with q/k/v and gate/up each one
-product; the steps between them are one hexkv launch each (residual sum and
-RMSNorm, head split and rotary, SwiGLU), and every KV byte moves through hexkv.
+product (joined once when the host is built, which takes about 1.3 times as
+long for it); the steps between them are one hexkv launch each (residual sum
+and RMSNorm, head split and rotary, SwiGLU).  For one or two tokens the
+products are hexkv's too (``ops.norm_linear``, ``ops.norm_rope_linear``), with
+the norm before and the rotary or SwiGLU after them in the same launch.  Every
+KV byte moves through hexkv.
 """
 from __future__ import annotations
 

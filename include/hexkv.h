@@ -48,8 +48,8 @@ enum hexkv_dtype {
 };
 
 /* Attention kernels.  AUTO picks TILES for 16-bit data with head_dim 64 or
- * 128 and q_len > 1 unless the call is small (few rows or keys, by max_seqlen),
- * else MFMA for such data with 8+ query heads per KV head, VALU otherwise; a work list is planned and launched with
+ * 128 and q_len > 1 unless the call is small (few rows or keys, by max_seqlen;
+ * an explicit partition is never small), else MFMA for such data with 8+ query heads per KV head, VALU otherwise; a work list is planned and launched with
  * hexkv_attend_plan_kernel's choice, which is ROWS for AUTO on large calls. */
 enum hexkv_kernel {
   HEXKV_KERNEL_AUTO = 0,
@@ -318,7 +318,8 @@ typedef struct hexkv_attend_layer {
  * overlap share launches: work lists planned for the XCDs (work_xcds > 0),
  * as many layers a launch as the arrival counters and the workspace hold.
  * Any other call, or layers_dev NULL, or a list of more than 1024 items, is
- * n_layers launches.
+ * n_layers launches.  Every layer's q must be there before the call: a step
+ * whose queries depend on the layer before (a decoder's) calls hexkv_attend.
  * hexkv_attend_layers_workspace_bytes returns the workspace that lets the
  * most layers share (never above 256 MiB for several); hexkv_attend's for
  * one layer is the least.  No counterpart in the reference.

@@ -1,5 +1,7 @@
-"""The query-tile attention kernel (q_len > 1, 16-bit, head_dim 64 / 128)
-against the float64 oracle, at the edges of its tiles.
+"""Attention of several query rows (q_len > 1, 16-bit, head_dim 64 / 128)
+against the float64 oracle, at the edges of the query-tile kernel's tiles.  An
+explicit partition takes that kernel at any size (4096: keys unsplit); without
+one small calls run the per-row kernels.
 
 Tolerances as for decode attention (max-abs, fp16 2e-3, bf16 8e-3): the
 output's own rounding plus fp32 sums of hi + lo probabilities (2^-17 relative
