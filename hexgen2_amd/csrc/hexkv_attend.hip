@@ -1579,12 +1579,19 @@ static int base_partition(const hexkv_attend_params *p) {
 // Measured per call with the merge, 192 and 128: Llama-2-7B 1 x 8192 28.4
 // and 39.1 us, 8 x 2048 46.5 and 54.0, 8 x 256-2048 25.5 and 26.9;
 // Llama-3-8B 16 x 128-2048 23.1 and 24.9, 1 x 8192 14.4 and 16.1; TinyLlama
-// 32 x 512-4096 25.0 and 27.6.  Below a want of 16 or 1024 positions 128
-// leads (Llama-2-7B 4 x 100-700: 10.4 and 10.9; TinyLlama 1 x 2048: 6.6 and
-// 7.3).
+// 32 x 512-4096 25.0 and 27.6.  Below a want of 16 128 leads (Llama-2-7B 4 x
+// 100-700: 10.4 and 10.9; TinyLlama 1 x 2048: 6.6 and 7.3).  Over 600 random
+// ragged calls (16 geometries, the three data types) 192 takes 0.935 of 128's
+// time in the geometric mean on rows of more than 1536 positions and heads of
+// up to 256 bytes; 17 of those 384 take over 1.05 times, at most 1.14.
+// Between 1280 and 1536 positions it gains nothing (1.01, up to 1.22), nor
+// for wider heads, whose workgroups are few and long (fp32 heads of 128: 0.99
+// and up to 1.27, of 256: 1.06 and up to 1.29).
 static int choose_partition(const hexkv_attend_params *p) {
   const int part = base_partition(p);
-  if (p->partition == 0 && p->q_len == 1 && part == 128 && p->max_seqlen > 1024 && wanted_partition(p) >= 16) return 192;
+  const bool narrow = static_cast<int64_t>(p->head_dim) * elem_size(p->dtype) <= 256;
+  if (p->partition == 0 && p->q_len == 1 && part == 128 && narrow && p->max_seqlen > 1536 && wanted_partition(p) >= 16)
+    return 192;
   return part;
 }
 

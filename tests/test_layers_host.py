@@ -176,3 +176,24 @@ def test_overlapping_outputs_are_refused(clash, call):
     rc = call(lib)
     assert (rc == _lib.HEXKV_EINVAL) == clash, lib.hexkv_last_error()
     assert not clash or b"overlap" in lib.hexkv_last_error()
+
+
+@pytest.mark.skipif(torch.cuda.device_count() > 0, reason="calls whose workspace fits would run on made-up addresses")
+@pytest.mark.parametrize("dtype,d,batch,longest,part", [
+    (0, 128, 8, 2048, 192), (1, 64, 16, 1537, 192), (2, 64, 16, 2048, 192),
+    (0, 128, 8, 1536, 128),                           # rows too short
+    (2, 128, 8, 2048, 128), (1, 256, 8, 2048, 128),   # heads of 512 bytes
+    (0, 128, 1, 2048, 128)])                          # too small a call
+def test_decode_partition(dtype, d, batch, longest, part):
+    """The partition a decode call runs with, by the workspace it accepts (one
+    that is large enough is then refused for its alignment)."""
+    lib = _lib.load()
+    heads = 8
+    p = _lib.AttendParams(dtype=dtype, batch=batch, q_len=1, q_heads=heads, kv_heads=heads, head_dim=d, q=256, cache=256,
+                          out=256, softmax_scale=1.0, capacity=longest, max_seqlen=longest, seqlen_bias=longest,
+                          q_batch_stride=heads * d, out_batch_stride=heads * d,
+                          cache_batch_stride=longest * 2 * heads * d, cache_pos_stride=2 * heads * d,
+                          cache_kv_stride=heads * d)
+    need = _lib.ATTEND_COUNTER_BYTES + batch * heads * -(-longest // part) * (d + 2) * 4
+    assert lib.hexkv_attend(p, 8, need - 1, None) == _lib.HEXKV_EWORKSPACE
+    assert lib.hexkv_attend(p, 8, need, None) == _lib.HEXKV_EINVAL
