@@ -1586,7 +1586,8 @@ static int base_partition(const hexkv_attend_params *p) {
 // up to 256 bytes; 17 of those 384 take over 1.05 times, at most 1.14.
 // Between 1280 and 1536 positions it gains nothing (1.01, up to 1.22), nor
 // for wider heads, whose workgroups are few and long (fp32 heads of 128: 0.99
-// and up to 1.27, of 256: 1.06 and up to 1.29).
+// and up to 1.27, of 256: 1.06 and up to 1.29).  500 calls over FT caches give
+// the same lines.
 static int choose_partition(const hexkv_attend_params *p) {
   const int part = base_partition(p);
   const bool narrow = static_cast<int64_t>(p->head_dim) * elem_size(p->dtype) <= 256;
@@ -2130,8 +2131,14 @@ static bool layers_independent(const hexkv_attend_params *p, const hexkv_attend_
 // 768 positions, 135.4 at 384; Llama-2-7B (4 of 122 MB) 79-84 at 128-256
 // against 88.7 at 112; Llama-3-8B with 8 rows (4 of 31 MB) 27.2-29.2 with
 // row blocks at 128-256, 32.7 with one head per item.
+// Row blocks need two segments (row, head block) per XCD: a segment's items
+// share one XCD, so with fewer the others idle.  Over 300 random geometries
+// row blocks take 0.97 of one-head items' time from 16 segments on, 1.06 with
+// 8-15, 1.4 with 4-7 and 2-3.4 below (one row of 8 heads over 7570 keys, 6
+// layers: 162 and 35 us, 80 as one launch a layer).
 constexpr int64_t kSharedLayerBytes = INT64_C(512) << 20;
 constexpr int64_t kSharedItems = 512;
+constexpr int64_t kSharedSegmentsPerXcd = 2;
 
 }  // namespace hexkv
 
@@ -2154,8 +2161,13 @@ extern "C" int hexkv_attend_plan_layers(const hexkv_attend_params *p, const int3
   const int64_t row_bytes = 2 * static_cast<int64_t>(p->head_dim) * elem_size(p->dtype);
   const int64_t bytes = positions * p->kv_heads * row_bytes;
   const bool shared = n_layers > 1 && p->work_xcds >= 1 && p->work_xcds <= 8 && bytes < kSharedLayerBytes;
-  if (shared && p->kernel == HEXKV_KERNEL_AUTO && rows_block(p) && bytes * n_layers >= (INT64_C(64) << 20))
-    one.kernel = HEXKV_KERNEL_ROWS;
+  if (shared && p->kernel == HEXKV_KERNEL_AUTO && rows_block(p)) {
+    const int64_t segments = static_cast<int64_t>(p->batch) * (p->kv_heads / rows_block(p));
+    if (segments < kSharedSegmentsPerXcd * p->work_xcds)
+      one.kernel = use_mfma(p, kernel_group(p->q_heads / p->kv_heads)) ? HEXKV_KERNEL_MFMA : HEXKV_KERNEL_VALU;
+    else if (bytes * n_layers >= (INT64_C(64) << 20))
+      one.kernel = HEXKV_KERNEL_ROWS;
+  }
   one.partition = p->partition;
   const int c = plan_request(&one, lens, what);
   if (c < 0) return c;

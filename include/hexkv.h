@@ -49,7 +49,8 @@ enum hexkv_dtype {
 
 /* Attention kernels.  AUTO picks TILES for 16-bit data with head_dim 64 or
  * 128 and q_len > 1 unless the call is small (few rows or keys, by max_seqlen;
- * an explicit partition is never small), else MFMA for such data with 8+ query heads per KV head, VALU otherwise; a work list is planned and launched with
+ * an explicit partition is never small), else MFMA for such data with 8+ query
+ * heads per KV head, VALU otherwise; a work list is planned and launched with
  * hexkv_attend_plan_kernel's choice, which is ROWS for AUTO on large calls. */
 enum hexkv_kernel {
   HEXKV_KERNEL_AUTO = 0,
@@ -402,7 +403,8 @@ int hexkv_attend_plan_kernel(const hexkv_attend_params *p, const int32_t *lens, 
 
 /* Kernel and chunk to plan a list with that n_layers layers of a
  * hexkv_attend_layers call share: hexkv_attend_plan_kernel's and
- * hexkv_attend_plan_chunk's for one layer.  An explicit p->kernel or
+ * hexkv_attend_plan_chunk's for one layer, for several ROWS only where its
+ * segments fill the XCDs.  An explicit p->kernel or
  * p->partition is kept. */
 int hexkv_attend_plan_layers(const hexkv_attend_params *p, const int32_t *lens, int n_layers, int32_t *kernel,
                              int32_t *chunk);

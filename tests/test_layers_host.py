@@ -36,6 +36,18 @@ def test_plan_layers(dtype, hq, hkv, d, lens, layers):
     assert n.value % 8 == 0 and (layers == 1 or most.value <= 64)
 
 
+@pytest.mark.parametrize("hq,hkv,rows,kernel", [(8, 8, 1, "valu"), (8, 8, 15, "valu"), (8, 8, 16, "rows"),
+                                                (32, 32, 3, "valu"), (32, 32, 4, "rows"), (32, 8, 3, "valu"),
+                                                (32, 8, 4, "rows")])
+def test_shared_row_blocks_fill_the_xcds(hq, hkv, rows, kernel):
+    """A segment's items run on one XCD: row blocks only with two segments for each."""
+    lib = _lib.load()
+    p = _params(0, rows, hq, hkv, 128, 7570)
+    k, chunk = ctypes.c_int32(), ctypes.c_int32()
+    assert lib.hexkv_attend_plan_layers(p, (ctypes.c_int32 * rows)(*[7570] * rows), 6, k, chunk) == 0
+    assert k.value == _lib.KERNELS[kernel]
+
+
 def test_plan_layers_keeps_what_the_caller_chose():
     lib = _lib.load()
     p = _params(0, 2, 32, 32, 128, 4000, kernel=1)
